@@ -1,10 +1,10 @@
 // FLOP census of the rollout kernel's algorithm (host-only measurement program).
 //
-// Instantiates the device dynamics of spi_dyn.h with an operation-counting scalar and runs
+// Instantiates the device dynamics (spi_fwd.h over spi_dyn.h) with an operation-counting scalar and runs
 // a representative rollout on the host: the Go2 settles from a standing pose, then follows
 // per-joint sinusoidal PD targets (amplitude U[0.1, 0.4] rad, frequency U[0.5, 3] Hz).  It
 // prints the mean number of floating-point operations per control step of the fused
-// rollout (PD + motor model + ABA + contact + integration per sub-interval, plus the
+// rollout (PD + motor model + leg elimination, base solve, contact and integration per sub-interval, plus the
 // tracking cost), which is the algorithmic work unit behind the roofline figure.
 //
 // Counting rule: +, -, *, / one FLOP each (a fused multiply-add therefore counts two);
@@ -95,6 +95,7 @@ inline bool isfinite(CountF a) { return std::isfinite(a.v); }
 
 #define SPI_REAL_T census::CountF
 #include "spi_dyn.h"
+#include "spi_fwd.h"
 #include "spi_adj.h"
 
 #include <vector>
@@ -133,6 +134,8 @@ int main() {
     lp.kp_s[l] = CountF::input(1.f); lp.kd_s[l] = CountF::input(1.f); lp.fric[l] = CountF::input(0.1f);
   }
   for (int g = 0; g < 3; ++g) lp.motor[g] = CountF::input(20.f);
+  LaneParams lq = lp;                    // the rollout kernels' base: with the legs' axial mass
+  lq.base = base_with_legs(lp.base);
 
   const int n_traj = 8, settle = 50, steps = 50;   // 1 s of excitation per trajectory
   // segment records of the rollout kernels' layout cut from the excitation (runtime values):
@@ -166,7 +169,7 @@ int main() {
         CountF tau[12];
         control_torques(a, lp, act, st, tau);
         CountF ff[12];
-        physics_step(a, lp, st, tau, ff);
+        physics_step_elim(a, LaneRegs{lq, tau}, st, ff);
         if (t >= settle) {
           for (int f = 0; f < 4; ++f) contact_feet += (ff[3 * f + 2].v > 0.f);
           ++physics_steps;
