@@ -88,6 +88,7 @@ inline CountF trans(float x, const CountF& a) {
 }
 inline CountF sqrtf(CountF a) { return trans(std::sqrt(a.v), a); }
 inline CountF expf(CountF a) { return trans(std::exp(a.v), a); }
+inline CountF exp2f(CountF a) { return trans(std::exp2(a.v), a); }
 inline CountF sinf(CountF a) { return trans(std::sin(a.v), a); }
 inline CountF cosf(CountF a) { return trans(std::cos(a.v), a); }
 inline bool isfinite(CountF a) { return std::isfinite(a.v); }

@@ -34,11 +34,13 @@ template <> struct LegConst<double> { using type = double; };
 using LegReal = LegConst<Real>::type;
 
 // Constants of one leg in its hip frame at O.  Thigh and calf: p, q = (Sxx +- Szz) / 2 and the
-// products of S about their axis, h the first moment; hip link: see above.
+// products of S about their axis (a 2 marks twice the value), h the first moment; hip link: see
+// above.
 template <class T> struct LegC {
-  T rx, ry, dz;                             // hip origin in the base, calf axis below O
-  T cp, cq, cxz, cxy, cyz, chx, chz, ci;    // calf; ci = 1 / (2 cp), its inverse joint inertia
-  T tp, tq, txz, txy, tyz, thx, thz;        // thigh, with the calf's axial mass
+  T rx, ry, sx, sy, dz;                     // hip origin in the base and its signs, calf axis below O
+  T cp, cp2, cq2, cxz2, cxy, cyz, chx, chz, ci;   // calf; ci = 1 / cp2, its inverse joint inertia
+  T tcp, tq2, txz2, txy, tyz, thx, thz;           // thigh, with the calf's axial mass; tcp = tp + cp
+  T d2;                                           // 2 (tp + cp) - 2 cp2: thigh pivot at n3 = 0
   T hhy, hhz, hyy, hzz, hxy, hxz, hyz;      // hip link, with the thigh's axial mass
   T fx, fy, fz;                             // foot sphere centre in the calf (y from O)
 };
@@ -76,9 +78,11 @@ template <class T> constexpr LegC<T> leg_c(int l) {
   const LegMass g = leg_mass(l);
   const double cp = 0.5 * (g.calf.xx + g.calf.zz), cq = 0.5 * (g.calf.xx - g.calf.zz);
   const double tp = 0.5 * (g.thigh.xx + g.thigh.zz), tq = 0.5 * (g.thigh.xx - g.thigh.zz);
-  return LegC<T>{T(g.rx), T(g.ry), T(g.dz),
-                 T(cp), T(cq), T(g.calf.xz), T(g.calf.xy), T(g.calf.yz), T(g.calf.hx), T(g.calf.hz), T(0.5 / cp),
-                 T(tp), T(tq), T(g.thigh.xz), T(g.thigh.xy), T(g.thigh.yz), T(g.thigh.hx), T(g.thigh.hz),
+  return LegC<T>{T(g.rx), T(g.ry), T(g.rx < 0 ? -1 : 1), T(g.ry < 0 ? -1 : 1), T(g.dz),
+                 T(cp), T(2.0 * cp), T(2.0 * cq), T(2.0 * g.calf.xz), T(g.calf.xy), T(g.calf.yz), T(g.calf.hx),
+                 T(g.calf.hz), T(0.5 / cp),
+                 T(tp + cp), T(2.0 * tq), T(2.0 * g.thigh.xz), T(g.thigh.xy), T(g.thigh.yz), T(g.thigh.hx),
+                 T(g.thigh.hz), T(2.0 * (tp + cp) - 4.0 * cp),
                  T(g.hip.hy), T(g.hip.hz), T(g.hip.yy), T(g.hip.zz), T(g.hip.xy), T(g.hip.xz), T(g.hip.yz),
                  T(SPI_FOOT_POS[3 * l]), T(SPI_FOOT_POS[3 * l + 1] + SPI_JOINT_ORIGIN[9 * l + 4]),
                  T(SPI_FOOT_POS[3 * l + 2])};
@@ -106,6 +110,21 @@ SPI_HD BaseInertia base_with_legs(const BaseInertia& b) {
                      b.ixz, b.iyz};
 }
 
+// 1 / (1 + 2^x): both tanh laws in one exponential and one reciprocal, with no sign handling:
+// 1 - tanh(u) = 2 / (1 + 2^(2 u log2 e)).  Its absolute error is spi_tanh's.
+SPI_HD Real spi_fall(Real x) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x));
+#else
+  return 1.0f / (1.0f + exp2f(x));
+#endif
+}
+constexpr float kTwoLog2e = 2.8853900817779268f;
+// tau - fric tanh(qd / v0) with inv = 2 log2(e) / v0.
+SPI_HD Real joint_friction(Real tau, Real fric, Real qd, Real inv) {
+  return (tau - fric) + 2.0f * fric * spi_fall(qd * inv);
+}
+
 // What the acceleration pass needs of a leg: the eliminated rows over their pivots (hip: n_y,
 // n_z, f; thigh, calf: n_z, f_x, f_z), the multipliers, the bias accelerations, the hip angle.
 struct LegElim {
@@ -130,93 +149,134 @@ SPI_HD void end_leg(ABI& I, F6& p) {
 #endif
 }
 
-// What the four legs share of the base state.
+// What the four legs share of the base state.  Products with the hip origin's coordinates carry
+// the sign-free |rx|, |ry| that all four legs have: a leg adds or subtracts them.
 struct BaseMotion {
   V3 w, v;        // base twist, base coordinates
   V3 up;          // world z in base coordinates
   Real z;         // base height
+  Real upx, upy;  // |rx| up.x, |ry| up.y
+  V3 cx, cy;      // w x (w x .) of (|rx|, 0, 0) and (0, |ry|, 0)
+  V3 wh;          // w x (w x h), h the base's first moment
 };
+constexpr LegReal kHipX = LegReal(SPI_JOINT_ORIGIN[0] < 0 ? -SPI_JOINT_ORIGIN[0] : SPI_JOINT_ORIGIN[0]);
+constexpr LegReal kHipY = LegReal(SPI_JOINT_ORIGIN[1] < 0 ? -SPI_JOINT_ORIGIN[1] : SPI_JOINT_ORIGIN[1]);
+constexpr bool hips_are_mirrored() {
+  for (int l = 0; l < 4; ++l)
+    for (int k = 0; k < 2; ++k)
+      if (SPI_JOINT_ORIGIN[9 * l + k] != SPI_JOINT_ORIGIN[k] && SPI_JOINT_ORIGIN[9 * l + k] != -SPI_JOINT_ORIGIN[k])
+        return false;
+  return true;
+}
+static_assert(hips_are_mirrored(), "the legs share the hip coordinates' magnitudes");
+SPI_HD BaseMotion base_motion(V3 w, V3 v, V3 up, Real z, const BaseInertia& B) {
+  const Real xx = w.x * w.x, yy = w.y * w.y, zz = w.z * w.z, xy = w.x * w.y, xz = w.x * w.z, yz = w.y * w.z;
+  const Real a = -(yy + zz), b = -(xx + zz), c = -(xx + yy);
+  return BaseMotion{w, v, up, z, kHipX * up.x, kHipY * up.y, V3{kHipX * a, kHipX * xy, kHipX * xz},
+                    V3{kHipY * xy, kHipY * b, kHipY * yz},
+                    V3{a * B.hx + xy * B.hy + xz * B.hz, xy * B.hx + b * B.hy + yz * B.hz,
+                       xz * B.hx + yz * B.hy + c * B.hz}};
+}
+
+// Joint angles' sine and cosine: the hardware's (1.2e-7 absolute), or exact to rounding.
+template <bool EXACT> SPI_HD void joint_sincos(Real x, Real* s, Real* c) {
+  if constexpr (EXACT) {
+    *s = sinf(x);
+    *c = cosf(x);
+  } else {
+    spi_sincos(x, s, c);
+  }
+}
+// a b + c in one rounding, in this order whatever the build lets the compiler regroup.
+SPI_HD Real spi_fma(Real a, Real b, Real c) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_fmaf(a, b, c);
+#else
+  return a * b + c;
+#endif
+}
 
 // Contact force of the foot sphere in the hip frame and its moments: about O (x, z), about the
 // thigh axis (y2) and the calf axis (y3).  The law of foot_contact (spi_dyn.h) with the normal
-// and the tangential velocity taken along the ground normal n instead of in world axes.
+// and the tangential velocity taken along the ground normal n instead of in world axes.  The
+// penetration is summed from the largest terms down: they cancel to the millimetre, and the
+// stiffness turns each 1e-8 m of rounding into 5e-4 N.
+// SKIP: lanes off the ground skip the block.  One rollout per lane, a wave holds candidates of one
+// segment, whose foot is off the ground together (4096 x 256 x H 20: 16.3 ms, 17.1 without the
+// branch); four lanes per rollout, a wave nearly always has a foot down and the skip only costs
+// its zeroed results (256 x 64 x H 5: 131 us, 126 without).
 struct FootLoad { V3 f; Real mx, mz, y2, y3; };
-template <class C>
+template <bool SKIP, class C>
 SPI_HD FootLoad foot_load(const SpiSimArgs& a, const C& k, const BaseMotion& b, Real x1, Real wy, Real wz, Real sd2,
                           Real sd3, Real c1, Real s1, Real dx, Real dz, Real c3, Real s3) {
   constexpr LegReal rad = LegReal(SPI_FOOT_RADIUS[0]);
-  const Real o(0.f);
+  const Real o(0.0f);
   FootLoad out{V3{o, o, o}, o, o, o, o};
   const V3 n = rotT<0>(b.up, c1, s1);
   const Real ex = c3 * k.fx + s3 * k.fz, ez = c3 * k.fz - s3 * k.fx;   // sphere centre from the calf axis
   const Real px = dx + ex, pz = dz + ez;
-  const Real height = b.z + (b.up.x * k.rx + b.up.y * k.ry) + (n.x * px + n.y * k.fy + n.z * pz);
-  const Real pen = rad - height;
-  if (pen > 0.0f) {
-    const Real qx = px - rad * n.x, qy = k.fy - rad * n.y, qz = pz - rad * n.z;   // contact point from O
-    const Real gx = ex - rad * n.x, gz = ez - rad * n.z;                          // ... from the calf axis
-    // velocity of that point of the calf: hip origin, hip rotation, the two spins about y
-    V3 v{b.v.x - b.w.z * k.ry, b.v.y + b.w.z * k.rx, b.v.z + (b.w.x * k.ry - b.w.y * k.rx)};
-    v = rotT<0>(v, c1, s1);
-    const Real y2 = wy + sd2;
-    v.x += y2 * qz - wz * qy + sd3 * gz;
-    v.y += wz * qx - x1 * qz;
-    v.z += x1 * qy - y2 * qx - sd3 * gx;
-    const Real vn = v.x * n.x + v.y * n.y + v.z * n.z;
-    const Real kpen = a.k_contact * pen;
-    const Real fn = kpen - kpen * spi_tanh(a.c_contact * vn * spi_rcp(kpen));
-    const V3 vt{v.x - vn * n.x, v.y - vn * n.y, v.z - vn * n.z};
-    const Real vt2 = vt.x * vt.x + vt.y * vt.y + vt.z * vt.z;
-    Real sc(0.0f);
-    if (vt2 > 0.0f) {
-      const Real inv = spi_rsqrt(vt2);
-      const Real t = vt2 * inv;
-      sc = fminf(a.c_tangent * t, a.mu * fn) * inv;
-    }
-    const V3 f{fn * n.x - sc * vt.x, fn * n.y - sc * vt.y, fn * n.z - sc * vt.z};
-    out.f = f;
-    out.mx = qy * f.z - qz * f.y;
-    out.mz = qx * f.y - qy * f.x;
-    out.y2 = qz * f.x - qx * f.z;
-    out.y3 = gz * f.x - gx * f.z;
-  }
+  const Real pen = -(spi_fma(n.z, pz, b.z - rad) + (n.x * px + n.y * k.fy + (k.sx * b.upx + k.sy * b.upy)));
+  if (SKIP && !(pen > Real(0.0f))) return out;
+  const Real qx = px - rad * n.x, qy = k.fy - rad * n.y, qz = pz - rad * n.z;   // contact point from O
+  const Real gx = ex - rad * n.x, gz = ez - rad * n.z;                          // ... from the calf axis
+  // velocity of that point of the calf: hip origin, hip rotation, the two spins about y
+  V3 v{b.v.x - b.w.z * k.ry, b.v.y + b.w.z * k.rx, b.v.z + (b.w.x * k.ry - b.w.y * k.rx)};
+  v = rotT<0>(v, c1, s1);
+  const Real y2 = wy + sd2;
+  v.x += y2 * qz - wz * qy + sd3 * gz;
+  v.y += wz * qx - x1 * qz;
+  v.z += x1 * qy - y2 * qx - sd3 * gx;
+  const Real vn = v.x * n.x + v.y * n.y + v.z * n.z;
+  const Real kpen = SKIP ? a.k_contact * pen : fmaxf(a.k_contact * pen, Real(1e-20f));
+  Real fn = 2.0f * kpen * spi_fall(a.c_contact * kTwoLog2e * vn * spi_rcp(kpen));
+  if (!SKIP) fn = pen > Real(0.0f) ? fn : o;   // and with it the friction cone and the force
+  const V3 vt{v.x - vn * n.x, v.y - vn * n.y, v.z - vn * n.z};
+  // min(c_t |vt|, mu fn) / |vt|; the 1e-30 (m/s)^2 keeps a foot at rest finite
+  const Real inv = spi_rsqrt(vt.x * vt.x + vt.y * vt.y + vt.z * vt.z + Real(1e-30f));
+  const Real sc = fminf(Real(a.c_tangent), a.mu * fn * inv);
+  const V3 f{fn * n.x - sc * vt.x, fn * n.y - sc * vt.y, fn * n.z - sc * vt.z};
+  out.f = f;
+  out.mx = qy * f.z - qz * f.y;
+  out.mz = qx * f.y - qy * f.x;
+  out.y2 = qz * f.x - qx * f.z;
+  out.y3 = gz * f.x - gx * f.z;
   return out;
 }
 
 // One leg: its articulated inertia and bias at the base origin (for the base solve, to be added
 // to the base's own) and the record for leg_resolve.  q, qd, tau: hip, thigh, calf (tau after
 // friction).  fout (optional): world contact force, R the base rotation.
-template <class C>
+template <bool SKIP, bool EXACT, class C>
 SPI_HD void leg_eliminate(const SpiSimArgs& a, const C& k, const BaseMotion& b, const Real* q, const Real* qd,
                           const Real* tau, ABI& Iout, F6& pout, LegElim& e, const G3* R, Real* fout) {
   Real c1, s1, c2, s2, c3, s3;
-  spi_sincos(q[0], &s1, &c1);
-  spi_sincos(q[1], &s2, &c2);
-  spi_sincos(q[1] + q[2], &s3, &c3);
+  joint_sincos<EXACT>(q[0], &s1, &c1);
+  joint_sincos<EXACT>(q[1], &s2, &c2);
+  joint_sincos<EXACT>(q[1] + q[2], &s3, &c3);
   const Real sd1 = qd[0], sd2 = qd[1], sd3 = qd[2];
 
-  // --- moments in the hip frame: calf about its axis (h, S), thigh + calf about O (g, T)
+  // --- moments in the hip frame: calf about its axis (h, S), thigh + calf about O (g, T);
+  // double angles as cos(2x) / 2 = c^2 - 1/2 and sin(2x) / 2 = c s
   const Real dx = k.dz * s2, dz = k.dz * c2;
-  const Real C2 = c3 * c3 - s3 * s3, S2 = 2.0f * (c3 * s3);
-  const Real ct = k.cq * C2 + k.cxz * S2;
+  const Real Cc = c3 * c3 - 0.5f, Sc = c3 * s3, Ct = c2 * c2 - 0.5f, St = c2 * s2;
   const Real hx = k.chx * c3 + k.chz * s3, hz = k.chz * c3 - k.chx * s3;
-  const Real Sxx = k.cp + ct, Szz = k.cp - ct, Sxz = k.cxz * C2 - k.cq * S2;
-  const Real Sxy = k.cxy * c3 + k.cyz * s3, Syz = k.cyz * c3 - k.cxy * s3;
-  const Real T2 = c2 * c2 - s2 * s2, U2 = 2.0f * (c2 * s2);
-  const Real tt = k.tq * T2 + k.txz * U2;
-  const Real dxhx = dx * hx, dzhz = dz * hz;
   const Real gx = k.thx * c2 + k.thz * s2 + hx, gz = k.thz * c2 - k.thx * s2 + hz;
-  const Real Txx = k.tp + tt + Sxx + 2.0f * dxhx, Tzz = k.tp - tt + Szz + 2.0f * dzhz;
-  const Real Txz = k.txz * T2 - k.tq * U2 + Sxz + dx * hz + dz * hx;
+  const Real ct = k.cq2 * Cc + k.cxz2 * Sc;
+  const Real Sxx = k.cp + ct, Szz = k.cp - ct, Sxz = k.cxz2 * Cc - k.cq2 * Sc;
+  const Real Sxy = k.cxy * c3 + k.cyz * s3, Syz = k.cyz * c3 - k.cxy * s3;
+  const Real tt = k.tq2 * Ct + k.txz2 * St + ct;
+  const Real dxhx = dx * hx, dzhz = dz * hz;
+  const Real Txx = 2.0f * dxhx + (k.tcp + tt), Tzz = 2.0f * dzhz + (k.tcp - tt);
+  const Real Txz = k.txz2 * Ct - k.tq2 * St + Sxz + dx * hz + dz * hx;
   const Real Txy = k.txy * c2 + k.tyz * s2 + Sxy, Tyz = k.tyz * c2 - k.txy * s2 + Syz;
   // whole leg about O: h = (gx, hhy, Hz), Sxx = Txx, Syy = hyy
   const Real Hz = gz + k.hhz, Vzz = Tzz + k.hzz, Vxy = Txy + k.hxy, Vxz = Txz + k.hxz, Vyz = Tyz + k.hyz;
 
   // --- elimination of the joint rows, calf first (its pivot is a constant)
-  const Real n3 = 2.0f * k.cp + dxhx + dzhz;           // calf row: n = (-Sxy, n3, -Syz), f = (hz, 0, -hx)
+  const Real n3 = k.cp2 + dxhx + dzhz;           // calf row: n = (-Sxy, n3, -Syz), f = (hz, 0, -hx)
   const Real l23 = n3 * k.ci, l13 = -k.ci * Sxy;
   const Real w3z = -k.ci * Syz, w3fx = k.ci * hz, w3fz = -k.ci * hx;
-  const Real D2 = Txx + Tzz - l23 * n3;
+  const Real D2 = k.d2 + 2.0f * n3 - l23 * n3;          // Txx + Tzz less the calf's share
   const Real H12 = l23 * Sxy - Txy;
   const Real F2z = l23 * Syz - Tyz, F2x = gz - l23 * hz, F2w = l23 * hx - gx;   // n_z, f_x, f_z
   const Real i2 = spi_rcp(D2);
@@ -240,11 +300,8 @@ SPI_HD void leg_eliminate(const SpiSimArgs& a, const C& k, const BaseMotion& b, 
   // --- velocity products: hip field A about O, spins of the thigh and calf on top
   const V3 w = rotT<0>(b.w, c1, s1);
   const Real x1 = w.x + sd1, x2 = x1 + sd1;
-  V3 aO;
-  {
-    const Real t = b.w.x * k.rx + b.w.y * k.ry, ww = dot(b.w, b.w);
-    aO = rotT<0>(V3{b.w.x * t - k.rx * ww, b.w.y * t - k.ry * ww, b.w.z * t}, c1, s1);
-  }
+  const V3 aO = rotT<0>(V3{k.sx * b.cx.x + k.sy * b.cy.x, k.sx * b.cx.y + k.sy * b.cy.y, k.sx * b.cx.z + k.sy * b.cy.z},
+                        c1, s1);
   const Real xx = x1 * x1, yy = w.y * w.y, zz = w.z * w.z;
   const Real Axx = -(yy + zz), Ayy = -(xx + zz), Azz = -(xx + yy);
   const Real Axy = w.y * x2, Axz = w.z * x2, Ayx = w.y * w.x, Azx = w.z * w.x, Ayz = w.y * w.z;   // Azy = Ayz
@@ -253,11 +310,12 @@ SPI_HD void leg_eliminate(const SpiSimArgs& a, const C& k, const BaseMotion& b, 
   const Real k3 = -(sd3 * (2.0f * y2 + sd3)), bx3 = 2.0f * (sd3 * x1), bz3 = 2.0f * (sd3 * w.z);
   const Real f3y = bx3 * hx + bz3 * hz;
   const Real dA = Axx - Azz;
-  const FootLoad fc = foot_load(a, k, b, x1, w.y, w.z, sd2, sd3, c1, s1, dx, dz, c3, s3);
+  const FootLoad fc = foot_load<SKIP>(a, k, b, x1, w.y, w.z, sd2, sd3, c1, s1, dx, dz, c3, s3);
   V3 f;
-  f.x = Axx * gx + Axy * k.hhy + Axz * Hz + k2 * gx + k3 * hx - fc.f.x;
+  const Real Bxx = Axx + k2, Bzz = Azz + k2;
+  f.x = Bxx * gx + Axy * k.hhy + Axz * Hz + k3 * hx - fc.f.x;
   f.y = Ayx * gx + Ayy * k.hhy + Ayz * Hz + bx2 * gx + bz2 * gz + f3y - fc.f.y;
-  f.z = Azx * gx + Ayz * k.hhy + Azz * Hz + k2 * gz + k3 * hz - fc.f.z;
+  f.z = Azx * gx + Ayz * k.hhy + Azz * k.hhz + Bzz * gz + k3 * hz - fc.f.z;
   const Real nx = k.hhy * aO.z - Hz * aO.y + Azx * Vxy + Ayz * (k.hyy - Vzz) + (Azz - Ayy) * Vyz - Ayx * Vxz +
                   (k2 * Tyz - bx2 * Txz - bz2 * Tzz) + (k3 * Syz - bx3 * Sxz - bz3 * Szz - dz * f3y) - fc.mx;
   const Real nz = gx * aO.y - k.hhy * aO.x + Ayx * Txx + (Ayy - Axx) * Vxy + Ayz * Vxz - Axy * k.hyy - Axz * Vyz +
@@ -265,7 +323,7 @@ SPI_HD void leg_eliminate(const SpiSimArgs& a, const C& k, const BaseMotion& b, 
   const Real nyh = k.hhz * aO.x + dA * k.hxz + Axz * k.hzz + Axy * k.hyz - Ayz * k.hxy;   // hip link alone
   const Real n2 = gz * aO.x - gx * aO.z + dA * Txz + Axz * Tzz - Azx * Txx + Axy * Tyz - Ayz * Txy +
                   k3 * (dz * hx - dx * hz) - fc.y2;
-  const Real acx = aO.x + (Axx + k2) * dx + Axz * dz, acz = aO.z + Azx * dx + (Azz + k2) * dz;
+  const Real acx = aO.x + Bxx * dx + Axz * dz, acz = aO.z + Azx * dx + Bzz * dz;
   const Real n3b = hz * acx - hx * acz + dA * Sxz + Axz * Szz - Azx * Sxx + Axy * Syz - Ayz * Sxy - fc.y3;
 
   const Real r3 = tau[2] - n3b, r2 = tau[1] - n2 - l23 * r3, r1 = tau[0] - nx - l13 * r3 - l12 * r2;
@@ -296,12 +354,10 @@ template <class C> SPI_HD void leg_resolve(const C& k, const LegElim& e, const M
 }
 
 // Base inertia blocks and velocity product of the base (with the legs' axial mass).
-SPI_HD void base_terms(const BaseInertia& B, V3 w, ABI& I, F6& p) {
+SPI_HD void base_terms(const BaseInertia& B, const BaseMotion& b, ABI& I, F6& p) {
   const RBT<Real> rb{B.m, B.hx, B.hy, B.hz, B.ixx, B.iyy, B.izz, B.ixy, B.ixz, B.iyz};
   I = rb_abi(rb);
-  const V3 h{B.hx, B.hy, B.hz};
-  p.n = cross(w, mul(I.A, w));
-  p.f = cross(w, cross(w, h));
+  p = F6{cross(b.w, mul(I.A, b.w)), b.wh};
 }
 // dv/dt of the base in base coordinates from its proper acceleration a0.
 SPI_HD M6 base_rate(const M6& a0, V3 w, V3 v, V3 up, Real g) {
@@ -309,7 +365,8 @@ SPI_HD M6 base_rate(const M6& a0, V3 w, V3 v, V3 up, Real g) {
 }
 
 // The lane's parameters and joint torques, all in registers.
-struct LaneRegs {
+template <bool EXACT = false> struct LaneRegsT {
+  static constexpr bool kSkip = false, kExact = EXACT;
   const LaneParams& lp;       // lp.base: base_with_legs()
   const Real* tau_motor;
   SPI_HD BaseInertia base() const { return lp.base; }
@@ -319,19 +376,21 @@ struct LaneRegs {
     *fric = lp.fric[l];
   }
 };
+using LaneRegs = LaneRegsT<false>;
 
 // forward_dynamics of spi_dyn.h by leg elimination.  P: base() the base inertia with the legs'
-// axial mass, leg(l, tau, &friction) the leg's motor torques and joint friction.
+// axial mass, leg(l, tau, &friction) the leg's motor torques and joint friction, kSkip of foot_load, kExact of joint_sincos.
 template <class P>
 SPI_HD void forward_dynamics_elim(const SpiSimArgs& a, const P& par, const State& st, M6& acc0, Real* qdd,
                                   Real* foot_force) {
   const G3 R = quat_to_rot(st.qx, st.qy, st.qz, st.qw);
-  const BaseMotion b{st.w, st.v, V3{R.m20, R.m21, R.m22}, st.p.z};
+  const BaseInertia B = par.base();
+  const BaseMotion b = base_motion(st.w, st.v, V3{R.m20, R.m21, R.m22}, st.p.z, B);
   constexpr LegC<LegReal> k0 = leg_c<LegReal>(0), k1 = leg_c<LegReal>(1), k2 = leg_c<LegReal>(2),
                           k3 = leg_c<LegReal>(3);
   ABI I;
   F6 p;
-  base_terms(par.base(), st.w, I, p);
+  base_terms(B, b, I, p);
   LegElim e[4];
 #define SPI_ELIM(L, K)                                                                                        \
   {                                                                                                           \
@@ -339,8 +398,9 @@ SPI_HD void forward_dynamics_elim(const SpiSimArgs& a, const P& par, const State
     F6 pt;                                                                                                    \
     Real tau[3], fric;                                                                                        \
     par.leg(L, tau, &fric);                                                                                   \
-    for (int j = 0; j < 3; ++j) tau[j] -= fric * spi_tanh(st.qd[3 * L + j] * a.fric_vel_inv);                 \
-    leg_eliminate(a, K, b, st.q + 3 * L, st.qd + 3 * L, tau, t, pt, e[L], &R,                                 \
+    for (int j = 0; j < 3; ++j)                                                                               \
+      tau[j] = joint_friction(tau[j], fric, st.qd[3 * L + j], a.fric_vel_inv * kTwoLog2e);                    \
+    leg_eliminate<P::kSkip, P::kExact>(a, K, b, st.q + 3 * L, st.qd + 3 * L, tau, t, pt, e[L], &R,                                 \
                   foot_force ? foot_force + 3 * L : nullptr);                                                 \
     abi_add(I, t);                                                                                            \
     p = F6{p.n + pt.n, p.f + pt.f};                                                                           \

@@ -6,8 +6,7 @@
 #include <cstring>
 
 #include "spi_dyn.h"
-#include "spi_dyn_leg.h"
-#include "spi_fwd.h"
+#include "spi_fwd_leg.h"
 #include "spi_launch.h"
 
 using namespace spi;
@@ -34,12 +33,12 @@ int launch_check(const char* what) { return hip_check(hipGetLastError(), what); 
 using spi_launch::apply_segment_gains;
 using spi_launch::xcd_remap;
 
-template <bool LEGS = true>
+// Parameters of lane i, the base with the legs' axial mass (spi_fwd.h).
 __device__ __forceinline__ LaneParams load_params(const float* __restrict__ par, int ld, int i) {
   LaneParams lp;
   lp.base = make_base_inertia(par[0 * ld + i], par[1 * ld + i], par[2 * ld + i], par[3 * ld + i], par[4 * ld + i],
                               par[5 * ld + i], par[6 * ld + i], par[7 * ld + i], par[8 * ld + i], par[9 * ld + i]);
-  if (LEGS) lp.base = base_with_legs(lp.base);
+  lp.base = base_with_legs(lp.base);
 #pragma unroll
   for (int l = 0; l < 4; ++l) {
     lp.kp_s[l] = par[(10 + l) * ld + i];
@@ -61,6 +60,7 @@ constexpr int kRolloutThreads = 256;
 // registers, the rollout fits the 256 that let two waves share a SIMD; the offset passes an
 // empty asm at each use so that the reads stay where they are.
 struct LaneLds {
+  static constexpr bool kSkip = true, kExact = false;
   static constexpr int kSlots = 10;   // base 3, legs 4 (tau, friction), kp_s, kd_s, motor
   float4* slot;                        // this thread's slot 0
   int stride;                          // threads per workgroup
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(kRolloutThreads) void rollout_cost_leg_kernel(
     if (l == 0) reinterpret_cast<unsigned int*>(out)[static_cast<size_t>(s) * n_cand + c] = 0x7f800000u;
     return;
   }
-  const LaneParams full = load_params<false>(par, ld, c);
+  const LaneParams full = load_params(par, ld, c);
   LegParams lp;
   lp.base = full.base;
   lp.kp_s = pick4(l, full.kp_s[0], full.kp_s[1], full.kp_s[2], full.kp_s[3]);
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(kRolloutThreads) void rollout_cost_leg_kernel(
   lp.fric = pick4(l, full.fric[0], full.fric[1], full.fric[2], full.fric[3]);
 #pragma unroll
   for (int g = 0; g < 3; ++g) lp.motor[g] = full.motor[g];
-  const LegK K = leg_constants(l);
+  const LegC<float> K = kElimTab.k[l];
   float kp[3], kd[3], q0[3], eff[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
@@ -203,7 +203,7 @@ __global__ __launch_bounds__(kRolloutThreads) void rollout_cost_leg_kernel(
     for (int d = 0; d < a.decimation; ++d) {
       float tau[3];
       control_torques_leg(a, lp, kp, kd, q0, eff, act, st.q, st.qd, tau);
-      physics_step_leg(a, lp, K, st, tau);
+      physics_step_elim_leg(a, lp, K, st, tau);
     }
     if (cost.mode == SPI_COST_TRACKING || t == H - 1) acc += step_cost_leg(cost, st, rec + 12, l);
     const float nrm = state_norm_leg(st);   // identical in the four lanes
@@ -268,55 +268,6 @@ __global__ __launch_bounds__(BLOCK, 2) void rollout_cost_batch_kernel(SpiSimArgs
       atomicExch(&queue[0], 0ULL);
       atomicExch(&queue[1], 0ULL);
     }
-  }
-}
-
-__global__ __launch_bounds__(256) void physics_step_kernel(SpiSimArgs a, const float* __restrict__ par, int ld,
-                                                           int n, float* __restrict__ root, float* __restrict__ dof,
-                                                           const float* __restrict__ torques,
-                                                           float* __restrict__ foot_force) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const LaneParams lp = load_params(par, ld, i);
-  State st;
-  float* r = root + static_cast<size_t>(i) * 13;
-  float* d = dof + static_cast<size_t>(i) * 24;
-  state_from_root(st, r, d, d + 1, 2);
-  float tau[12];
-#pragma unroll
-  for (int j = 0; j < 12; ++j) tau[j] = torques[static_cast<size_t>(i) * 12 + j];
-  float ff[12];
-  physics_step_elim(a, LaneRegs{lp, tau}, st, foot_force ? ff : nullptr);
-  state_to_root(st, r, d, d + 1, 2);
-  if (foot_force) {
-#pragma unroll
-    for (int k = 0; k < 12; ++k) foot_force[static_cast<size_t>(i) * 12 + k] = ff[k];
-  }
-}
-
-__global__ __launch_bounds__(256) void forward_dynamics_kernel(SpiSimArgs a, const float* __restrict__ par, int ld,
-                                                               int n, const float* __restrict__ root,
-                                                               const float* __restrict__ dof,
-                                                               const float* __restrict__ torques,
-                                                               float* __restrict__ acc, float* __restrict__ foot_force) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const LaneParams lp = load_params(par, ld, i);
-  State st;
-  state_from_root(st, root + static_cast<size_t>(i) * 13, dof + static_cast<size_t>(i) * 24,
-                  dof + static_cast<size_t>(i) * 24 + 1, 2);
-  float tau[12], qdd[12], ff[12];
-#pragma unroll
-  for (int j = 0; j < 12; ++j) tau[j] = torques[static_cast<size_t>(i) * 12 + j];
-  M6 a0;
-  forward_dynamics_elim(a, LaneRegs{lp, tau}, st, a0, qdd, foot_force ? ff : nullptr);
-  float* o = acc + static_cast<size_t>(i) * 18;
-  o[0] = a0.w.x; o[1] = a0.w.y; o[2] = a0.w.z; o[3] = a0.v.x; o[4] = a0.v.y; o[5] = a0.v.z;
-#pragma unroll
-  for (int j = 0; j < 12; ++j) o[6 + j] = qdd[j];
-  if (foot_force) {
-#pragma unroll
-    for (int k = 0; k < 12; ++k) foot_force[static_cast<size_t>(i) * 12 + k] = ff[k];
   }
 }
 
@@ -445,31 +396,6 @@ __global__ void fd_fim_kernel(const float* __restrict__ root, const float* __res
   for (int k = 0; k < g; ++k) out[im + k] = acc;
 }
 
-// Record mode: per-lane params, initial state and action sequence; state after every control step.
-__global__ __launch_bounds__(256) void simulate_kernel(SpiSimArgs a, const float* __restrict__ par, int ld, int n,
-                                                       const float* __restrict__ init,
-                                                       const float* __restrict__ actions, int T,
-                                                       float* __restrict__ states) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const LaneParams lp = load_params(par, ld, i);
-  State st;
-  const float* s0 = init + static_cast<size_t>(i) * SPI_STATE_DIM;
-  state_from_root(st, s0, s0 + 13, s0 + 25, 1);
-  for (int t = 0; t < T; ++t) {
-    float act[12];
-#pragma unroll
-    for (int j = 0; j < 12; ++j) act[j] = actions[(static_cast<size_t>(i) * T + t) * 12 + j];
-    for (int d = 0; d < a.decimation; ++d) {
-      float tau[12];
-      control_torques(a, lp, act, st, tau);
-      physics_step_elim(a, LaneRegs{lp, tau}, st, nullptr);
-    }
-    float* o = states + (static_cast<size_t>(i) * T + t) * SPI_STATE_DIM;
-    state_to_root(st, o, o + 13, o + 25, 1);
-  }
-}
-
 // Active-sysID FD-FIM rollout.  Group of G = n_param + 1 envs on G2 = pow2 >= G consecutive
 // lanes of one wavefront (padding lanes shadow the main env and contribute nothing); states
 // of the main env are read by the aux lanes with cross-lane shuffles.
@@ -570,29 +496,6 @@ extern "C" {
 const char* spi_last_error(void) { return g_err; }
 int spi_abi_version(void) { return SPI_ABI_VERSION; }
 int spi_segment_stride(int horizon) { return SPI_STATE_DIM + horizon * (12 + SPI_STATE_DIM); }
-
-int spi_physics_step(const SpiSimArgs* sim, const float* params_dev, int ld, int n, float* root_dev,
-                     float* dof_state_dev, const float* torques_dev, float* foot_force_dev, hipStream_t stream) {
-  if (!sim_args_ok(sim)) return fail(SPI_ERR_INVALID_ARG, "spi_physics_step: invalid SpiSimArgs");
-  if (n < 0 || ld < n || !params_dev || !root_dev || !dof_state_dev || !torques_dev)
-    return fail(SPI_ERR_INVALID_ARG, "spi_physics_step: bad sizes or null pointer");
-  if (n == 0) return SPI_OK;
-  physics_step_kernel<<<(n + 255) / 256, 256, 0, stream>>>(*sim, params_dev, ld, n, root_dev, dof_state_dev,
-                                                          torques_dev, foot_force_dev);
-  return launch_check("physics_step_kernel");
-}
-
-int spi_forward_dynamics(const SpiSimArgs* sim, const float* params_dev, int ld, int n, const float* root_dev,
-                         const float* dof_state_dev, const float* torques_dev, float* acc_dev, float* foot_force_dev,
-                         hipStream_t stream) {
-  if (!sim_args_ok(sim)) return fail(SPI_ERR_INVALID_ARG, "spi_forward_dynamics: invalid SpiSimArgs");
-  if (n < 0 || ld < n || !params_dev || !root_dev || !dof_state_dev || !torques_dev || !acc_dev)
-    return fail(SPI_ERR_INVALID_ARG, "spi_forward_dynamics: bad sizes or null pointer");
-  if (n == 0) return SPI_OK;
-  forward_dynamics_kernel<<<(n + 255) / 256, 256, 0, stream>>>(*sim, params_dev, ld, n, root_dev, dof_state_dev,
-                                                              torques_dev, acc_dev, foot_force_dev);
-  return launch_check("forward_dynamics_kernel");
-}
 
 int spi_set_rows_indexed(float* dst_dev, const float* src_dev, const int* idx_dev, int n_idx, int n_rows, int row_len,
                          hipStream_t stream) {
@@ -717,17 +620,6 @@ int spi_batch_rollout_cost(const SpiSimArgs* sim, const SpiBatchProblem* probs_d
   else return fail(SPI_ERR_INVALID_ARG, "spi_batch_rollout_cost: block must be 64/128/256, unroll 1/2");
 #undef SPI_BATCH_LAUNCH
   return launch_check("rollout_cost_batch_kernel");
-}
-
-int spi_simulate(const SpiSimArgs* sim, const float* params_dev, int ld, int n, const float* init_dev,
-                 const float* actions_dev, int n_steps, float* states_dev, hipStream_t stream) {
-  if (!sim_args_ok(sim)) return fail(SPI_ERR_INVALID_ARG, "spi_simulate: invalid SpiSimArgs");
-  if (n < 0 || ld < n || n_steps < 0 || !params_dev || !init_dev || !actions_dev || !states_dev)
-    return fail(SPI_ERR_INVALID_ARG, "spi_simulate: bad sizes or null pointer");
-  if (n == 0 || n_steps == 0) return SPI_OK;
-  simulate_kernel<<<(n + 255) / 256, 256, 0, stream>>>(*sim, params_dev, ld, n, init_dev, actions_dev, n_steps,
-                                                       states_dev);
-  return launch_check("simulate_kernel");
 }
 
 }  // extern "C"

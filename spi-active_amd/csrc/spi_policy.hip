@@ -12,8 +12,7 @@
 
 #include <cstdio>
 
-#include "spi_dyn.h"
-#include "spi_dyn_leg.h"
+#include "spi_fwd_leg.h"
 #include "spi_launch.h"
 
 using namespace spi;
@@ -39,10 +38,12 @@ __constant__ int kDim[kKeys] = {12, 3, 4, 1, 2, 1, 1, 1, 4, 2, 2, 12, 12, 3};
 constexpr int kOffHost[kKeys] = {0, 12, 15, 19, 20, 22, 23, 24, 25, 29, 31, 33, 45, 57};
 constexpr int kDimHost[kKeys] = {12, 3, 4, 1, 2, 1, 1, 1, 4, 2, 2, 12, 12, 3};
 
+// Parameters of env i, the base with the legs' axial mass (spi_fwd.h).
 __device__ __forceinline__ LaneParams load_lane(const float* __restrict__ par, int ld, int i) {
   LaneParams lp;
   lp.base = make_base_inertia(par[0 * ld + i], par[1 * ld + i], par[2 * ld + i], par[3 * ld + i], par[4 * ld + i],
                               par[5 * ld + i], par[6 * ld + i], par[7 * ld + i], par[8 * ld + i], par[9 * ld + i]);
+  lp.base = base_with_legs(lp.base);
 #pragma unroll
   for (int l = 0; l < 4; ++l) {
     lp.kp_s[l] = par[(10 + l) * ld + i];
@@ -104,7 +105,7 @@ __global__ __launch_bounds__(kPolThreads) void policy_step_kernel(SpiSimArgs a, 
     } else {
       control_torques(a, lp, act, st, tau);
     }
-    physics_step(a, lp, st, tau, nullptr);
+    physics_step_elim(a, LaneRegs{lp, tau}, st, nullptr);
   }
   const float nrm = state_norm(st);
   if (!finite_bits(nrm) || nrm >= a.state_limit) bad[i] = 1;
@@ -129,14 +130,15 @@ __global__ __launch_bounds__(kPolThreads) void policy_step_leg_kernel(SpiSimArgs
   const int i = t >> 2, l = t & 3;
   if (i >= n) return;  // the four lanes of an env leave together
   LegParams lp;
-  lp.base = make_base_inertia(par[0 * ld + i], par[1 * ld + i], par[2 * ld + i], par[3 * ld + i], par[4 * ld + i],
-                              par[5 * ld + i], par[6 * ld + i], par[7 * ld + i], par[8 * ld + i], par[9 * ld + i]);
+  lp.base = base_with_legs(make_base_inertia(par[0 * ld + i], par[1 * ld + i], par[2 * ld + i], par[3 * ld + i],
+                                             par[4 * ld + i], par[5 * ld + i], par[6 * ld + i], par[7 * ld + i],
+                                             par[8 * ld + i], par[9 * ld + i]));
   lp.kp_s = par[(10 + l) * ld + i];
   lp.kd_s = par[(14 + l) * ld + i];
   lp.fric = par[(18 + l) * ld + i];
 #pragma unroll
   for (int g = 0; g < 3; ++g) lp.motor[g] = par[(22 + g) * ld + i];
-  const LegK K = leg_constants(l);
+  const LegC<float> K = kElimTab.k[l];
   float kp[3], kd[3], q0[3], eff[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
@@ -168,7 +170,7 @@ __global__ __launch_bounds__(kPolThreads) void policy_step_leg_kernel(SpiSimArgs
     } else {
       control_torques_leg(a, lp, kp, kd, q0, eff, act, st.q, st.qd, tau);
     }
-    physics_step_leg(a, lp, K, st, tau);
+    physics_step_elim_leg(a, lp, K, st, tau);
   }
   const float nrm = state_norm_leg(st);
   if (l == 0 && (!finite_bits(nrm) || nrm >= a.state_limit)) bad[i] = 1;

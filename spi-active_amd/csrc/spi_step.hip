@@ -1,0 +1,158 @@
+// Single physics steps, forward dynamics and record mode (the states of a rollout after every
+// control step), one env per lane.  In a source of its own, so that a simulator's trajectories and
+// recorded data sets do not change in the last bit when a scoring kernel does.
+#include <hip/hip_runtime.h>
+
+#include <cstdio>
+
+#include "spi_fwd.h"
+
+using namespace spi;
+
+namespace {
+
+int rfail(int code, const char* msg) {
+  spi_set_error(msg);
+  return code;
+}
+
+// Parameters of lane i, the base with the legs' axial mass (spi_fwd.h).
+__device__ __forceinline__ LaneParams load_params(const float* __restrict__ par, int ld, int i) {
+  LaneParams lp;
+  lp.base = base_with_legs(make_base_inertia(par[0 * ld + i], par[1 * ld + i], par[2 * ld + i], par[3 * ld + i],
+                                             par[4 * ld + i], par[5 * ld + i], par[6 * ld + i], par[7 * ld + i],
+                                             par[8 * ld + i], par[9 * ld + i]));
+#pragma unroll
+  for (int l = 0; l < 4; ++l) {
+    lp.kp_s[l] = par[(10 + l) * ld + i];
+    lp.kd_s[l] = par[(14 + l) * ld + i];
+    lp.fric[l] = par[(18 + l) * ld + i];
+  }
+#pragma unroll
+  for (int g = 0; g < 3; ++g) lp.motor[g] = par[(22 + g) * ld + i];
+  return lp;
+}
+
+__global__ __launch_bounds__(256) void physics_step_kernel(SpiSimArgs a, const float* __restrict__ par, int ld,
+                                                           int n, float* __restrict__ root, float* __restrict__ dof,
+                                                           const float* __restrict__ torques,
+                                                           float* __restrict__ foot_force) {
+  int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const LaneParams lp = load_params(par, ld, i);
+  State st;
+  float* r = root + static_cast<size_t>(i) * 13;
+  float* d = dof + static_cast<size_t>(i) * 24;
+  state_from_root(st, r, d, d + 1, 2);
+  float tau[12];
+#pragma unroll
+  for (int j = 0; j < 12; ++j) tau[j] = torques[static_cast<size_t>(i) * 12 + j];
+  float ff[12];
+  physics_step_elim(a, LaneRegs{lp, tau}, st, foot_force ? ff : nullptr);
+  state_to_root(st, r, d, d + 1, 2);
+  if (foot_force) {
+#pragma unroll
+    for (int k = 0; k < 12; ++k) foot_force[static_cast<size_t>(i) * 12 + k] = ff[k];
+  }
+}
+
+__global__ __launch_bounds__(256) void forward_dynamics_kernel(SpiSimArgs a, const float* __restrict__ par, int ld,
+                                                               int n, const float* __restrict__ root,
+                                                               const float* __restrict__ dof,
+                                                               const float* __restrict__ torques,
+                                                               float* __restrict__ acc, float* __restrict__ foot_force) {
+  int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const LaneParams lp = load_params(par, ld, i);
+  State st;
+  state_from_root(st, root + static_cast<size_t>(i) * 13, dof + static_cast<size_t>(i) * 24,
+                  dof + static_cast<size_t>(i) * 24 + 1, 2);
+  float tau[12], qdd[12], ff[12];
+#pragma unroll
+  for (int j = 0; j < 12; ++j) tau[j] = torques[static_cast<size_t>(i) * 12 + j];
+  M6 a0;
+  // one evaluation, bound by its memory and launch: accurate angles cost it nothing
+  forward_dynamics_elim(a, LaneRegsT<true>{lp, tau}, st, a0, qdd, foot_force ? ff : nullptr);
+  float* o = acc + static_cast<size_t>(i) * 18;
+  o[0] = a0.w.x; o[1] = a0.w.y; o[2] = a0.w.z; o[3] = a0.v.x; o[4] = a0.v.y; o[5] = a0.v.z;
+#pragma unroll
+  for (int j = 0; j < 12; ++j) o[6 + j] = qdd[j];
+  if (foot_force) {
+#pragma unroll
+    for (int k = 0; k < 12; ++k) foot_force[static_cast<size_t>(i) * 12 + k] = ff[k];
+  }
+}
+
+// Record mode: per-lane params, initial state and action sequence; state after every control step.
+__global__ __launch_bounds__(256) void simulate_kernel(SpiSimArgs a, const float* __restrict__ par, int ld, int n,
+                                                       const float* __restrict__ init,
+                                                       const float* __restrict__ actions, int T,
+                                                       float* __restrict__ states) {
+  int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const LaneParams lp = load_params(par, ld, i);
+  State st;
+  const float* s0 = init + static_cast<size_t>(i) * SPI_STATE_DIM;
+  state_from_root(st, s0, s0 + 13, s0 + 25, 1);
+  for (int t = 0; t < T; ++t) {
+    float act[12];
+#pragma unroll
+    for (int j = 0; j < 12; ++j) act[j] = actions[(static_cast<size_t>(i) * T + t) * 12 + j];
+    for (int d = 0; d < a.decimation; ++d) {
+      float tau[12];
+      control_torques(a, lp, act, st, tau);
+      physics_step_elim(a, LaneRegs{lp, tau}, st, nullptr);
+    }
+    float* o = states + (static_cast<size_t>(i) * T + t) * SPI_STATE_DIM;
+    state_to_root(st, o, o + 13, o + 25, 1);
+  }
+}
+
+bool sim_args_ok(const SpiSimArgs* a) {
+  return a && a->dt > 0.f && a->decimation >= 1 && a->decimation <= 64 && a->substeps >= 1 && a->substeps <= 64 &&
+         a->motor_model >= 0 && a->motor_model <= 3 && a->state_limit > 0.f;
+}
+int launched() {
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? SPI_OK : rfail(SPI_ERR_HIP, hipGetErrorString(e));
+}
+
+}  // namespace
+
+extern "C" {
+
+int spi_physics_step(const SpiSimArgs* sim, const float* params_dev, int ld, int n, float* root_dev,
+                     float* dof_state_dev, const float* torques_dev, float* foot_force_dev, hipStream_t stream) {
+  if (!sim_args_ok(sim)) return rfail(SPI_ERR_INVALID_ARG, "spi_physics_step: invalid SpiSimArgs");
+  if (n < 0 || ld < n || !params_dev || !root_dev || !dof_state_dev || !torques_dev)
+    return rfail(SPI_ERR_INVALID_ARG, "spi_physics_step: bad sizes or null pointer");
+  if (n == 0) return SPI_OK;
+  physics_step_kernel<<<(n + 255) / 256, 256, 0, stream>>>(*sim, params_dev, ld, n, root_dev, dof_state_dev,
+                                                          torques_dev, foot_force_dev);
+  return launched();
+}
+
+int spi_forward_dynamics(const SpiSimArgs* sim, const float* params_dev, int ld, int n, const float* root_dev,
+                         const float* dof_state_dev, const float* torques_dev, float* acc_dev, float* foot_force_dev,
+                         hipStream_t stream) {
+  if (!sim_args_ok(sim)) return rfail(SPI_ERR_INVALID_ARG, "spi_forward_dynamics: invalid SpiSimArgs");
+  if (n < 0 || ld < n || !params_dev || !root_dev || !dof_state_dev || !torques_dev || !acc_dev)
+    return rfail(SPI_ERR_INVALID_ARG, "spi_forward_dynamics: bad sizes or null pointer");
+  if (n == 0) return SPI_OK;
+  forward_dynamics_kernel<<<(n + 255) / 256, 256, 0, stream>>>(*sim, params_dev, ld, n, root_dev, dof_state_dev,
+                                                              torques_dev, acc_dev, foot_force_dev);
+  return launched();
+}
+
+int spi_simulate(const SpiSimArgs* sim, const float* params_dev, int ld, int n, const float* init_dev,
+                 const float* actions_dev, int n_steps, float* states_dev, hipStream_t stream) {
+  if (!sim_args_ok(sim)) return rfail(SPI_ERR_INVALID_ARG, "spi_simulate: invalid SpiSimArgs");
+  if (n < 0 || ld < n || n_steps < 0 || !params_dev || !init_dev || !actions_dev || !states_dev)
+    return rfail(SPI_ERR_INVALID_ARG, "spi_simulate: bad sizes or null pointer");
+  if (n == 0 || n_steps == 0) return SPI_OK;
+  simulate_kernel<<<(n + 255) / 256, 256, 0, stream>>>(*sim, params_dev, ld, n, init_dev, actions_dev, n_steps,
+                                                       states_dev);
+  return launched();
+}
+
+}  // extern "C"

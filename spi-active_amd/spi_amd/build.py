@@ -19,7 +19,7 @@ CSRC = os.path.join(PKG_ROOT, "csrc")
 INCLUDE = os.path.join(REPO_ROOT, "include")
 LIB_DIR = os.path.join(PKG_ROOT, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libspi_hip.so")
-SOURCES = ["spi_kernels.hip", "spi_cem.hip", "spi_sens.hip", "spi_sens_lane.hip", "spi_sens_pair.hip",
+SOURCES = ["spi_kernels.hip", "spi_step.hip", "spi_cem.hip", "spi_sens.hip", "spi_sens_lane.hip", "spi_sens_pair.hip",
            "spi_fisher.hip",
            "spi_commands.hip", "spi_data.hip", "spi_adjoint.hip", "spi_adjoint_lane.hip", "spi_policy.hip",
            "spi_mlp.hip"]
@@ -34,7 +34,7 @@ SOURCES = ["spi_kernels.hip", "spi_cem.hip", "spi_sens.hip", "spi_sens_lane.hip"
 # CEM, the cost reduction and the Fisher/logdet kernels keep strict IEEE semantics.
 DYN_FLAGS = ["-ffinite-math-only"]
 DYN_REASSOC_FLAGS = DYN_FLAGS + ["-fassociative-math", "-DSPI_REASSOCIATE=1"]
-FILE_FLAGS = {"spi_kernels.hip": DYN_REASSOC_FLAGS, "spi_cem.hip": [], "spi_sens.hip": DYN_REASSOC_FLAGS,
+FILE_FLAGS = {"spi_kernels.hip": DYN_REASSOC_FLAGS, "spi_step.hip": DYN_REASSOC_FLAGS, "spi_cem.hip": [], "spi_sens.hip": DYN_REASSOC_FLAGS,
               "spi_sens_lane.hip": DYN_FLAGS,
               "spi_sens_pair.hip": DYN_REASSOC_FLAGS,
               "spi_fisher.hip": [], "spi_commands.hip": [], "spi_data.hip": [],
