@@ -32,9 +32,10 @@ from ..params import PARAM_NAMES
 from ..rollout import C_ref, RolloutEngine
 from .active import KSYNC_MODES, _alias
 
-# Up to this many envs the four-lanes-per-env physics runs faster (one env per lane leaves
-# SIMDs idle below ~64 K envs and has ~3x the instructions per lane on the critical path).
-LEG_PARALLEL_MAX_ENVS = 16384
+# Up to this many envs the four-lanes-per-env physics runs faster: one wave per SIMD carries 16,384
+# envs, one env per lane takes the time of one wave up to 65,536.  One control step, legs against
+# lanes: 32 / 73 us at 16,384 envs, 54 / 75 at 32,768, 74 / 76 at 40,960, 97 / 78 at 65,536.
+LEG_PARALLEL_MAX_ENVS = 32768
 OBS_TERMS = 60
 OBS_HISTORY = 14
 ACTOR_HIDDEN = (512, 256, 128)

@@ -19,10 +19,11 @@ DEFAULT_TRACKING_WEIGHTS = (10.0, 5.0, 1.0, 1.0, 1.0, 0.05)
 REFERENCE_WEIGHTS = (10.0, 5.0, 0.0, 0.0, 1.0, 0.0)
 
 
-# Up to this many (candidate, segment) rollouts the four-lanes-per-rollout kernel is faster:
-# one rollout per lane leaves SIMDs idle below ~64 K rollouts and has ~3x the instructions per
-# lane on the critical path.
-LEG_PARALLEL_MAX_ROLLOUTS = 16384
+# Up to this many (candidate, segment) rollouts the four-lanes-per-rollout kernel is faster.  Its
+# time goes by whole waves per SIMD (one per 16,384 rollouts), one rollout per lane takes the time
+# of one wave up to 65,536: H 10, legs against lanes 264 / 690 us at 16,384 rollouts, 456 / 688 at
+# 32,768, 650 / 690 at 49,152, 838 / 695 at 57,344.
+LEG_PARALLEL_MAX_ROLLOUTS = 49152
 
 
 class RolloutEngine:
