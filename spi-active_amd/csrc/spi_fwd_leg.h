@@ -14,11 +14,12 @@ struct ElimTable { LegC<float> k[4]; };
 constexpr ElimTable elim_table() { return ElimTable{{leg_c<float>(0), leg_c<float>(1), leg_c<float>(2), leg_c<float>(3)}}; }
 static __constant__ ElimTable kElimTab = elim_table();
 
-// forward_dynamics_elim, leg-parallel: k this lane's leg; lp.base is base_with_legs().  All four
-// lanes of a rollout must be active.
+// forward_dynamics_elim, leg-parallel: k this lane's leg; lp.base is base_with_legs(); foot_force
+// (optional) this leg's.  All four lanes of a rollout must be active.
 __device__ __forceinline__ void forward_dynamics_elim_leg(const SpiSimArgs& a, const LegParams& lp,
                                                           const LegC<float>& k, const LegState& st,
-                                                          const Real* tau_motor, M6& acc0, Real* qdd) {
+                                                          const Real* tau_motor, M6& acc0, Real* qdd,
+                                                          Real* foot_force = nullptr) {
   const G3 R = quat_to_rot(st.qx, st.qy, st.qz, st.qw);
   const BaseMotion b = base_motion(st.w, st.v, V3{R.m20, R.m21, R.m22}, st.p.z, lp.base);
   Real tau[3];
@@ -28,7 +29,7 @@ __device__ __forceinline__ void forward_dynamics_elim_leg(const SpiSimArgs& a, c
   ABI I, t;
   F6 p, pt;
   LegElim e;
-  leg_eliminate<false, false>(a, k, b, st.q, st.qd, tau, t, pt, e, &R, nullptr);
+  leg_eliminate<false, false>(a, k, b, st.q, st.qd, tau, t, pt, e, &R, foot_force);
   sum4(t);
   sum4(pt.n);
   sum4(pt.f);
@@ -40,12 +41,13 @@ __device__ __forceinline__ void forward_dynamics_elim_leg(const SpiSimArgs& a, c
 }
 
 __device__ __forceinline__ void physics_step_elim_leg(const SpiSimArgs& a, const LegParams& lp, const LegC<float>& k,
-                                                      LegState& st, const Real* tau_motor) {
+                                                      LegState& st, const Real* tau_motor,
+                                                      Real* foot_force = nullptr) {
   const Real h = a.dt / Real(a.substeps);
   for (int i = 0; i < a.substeps; ++i) {
     M6 acc0;
     Real qdd[3];
-    forward_dynamics_elim_leg(a, lp, k, st, tau_motor, acc0, qdd);
+    forward_dynamics_elim_leg(a, lp, k, st, tau_motor, acc0, qdd, foot_force);
     integrate_leg(st, acc0, qdd, h);
   }
 }

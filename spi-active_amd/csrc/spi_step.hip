@@ -5,7 +5,7 @@
 
 #include <cstdio>
 
-#include "spi_fwd.h"
+#include "spi_fwd_leg.h"
 
 using namespace spi;
 
@@ -53,6 +53,48 @@ __global__ __launch_bounds__(256) void physics_step_kernel(SpiSimArgs a, const f
   if (foot_force) {
 #pragma unroll
     for (int k = 0; k < 12; ++k) foot_force[static_cast<size_t>(i) * 12 + k] = ff[k];
+  }
+}
+
+// physics_step_kernel with four lanes per env, one per leg.  Up to kLegStepMaxEnvs: an env loop of a
+// few thousand envs is one wave's latency, and a leg's share of the step is a third of it (4096
+// envs 19 -> 9 us; one wave per SIMD carries 16,384 envs here and 65,536 above).
+constexpr int kLegStepMaxEnvs = 32768;
+__global__ __launch_bounds__(256) void physics_step_leg_kernel(SpiSimArgs a, const float* __restrict__ par, int ld,
+                                                               int n, float* __restrict__ root,
+                                                               float* __restrict__ dof,
+                                                               const float* __restrict__ torques,
+                                                               float* __restrict__ foot_force) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = t >> 2, l = t & 3;
+  if (i >= n) return;  // the four lanes of an env leave together
+  LegParams lp;
+  lp.base = base_with_legs(make_base_inertia(par[0 * ld + i], par[1 * ld + i], par[2 * ld + i], par[3 * ld + i],
+                                             par[4 * ld + i], par[5 * ld + i], par[6 * ld + i], par[7 * ld + i],
+                                             par[8 * ld + i], par[9 * ld + i]));
+  lp.fric = par[(18 + l) * ld + i];
+  LegState st;
+  float* r = root + static_cast<size_t>(i) * 13;
+  float* d = dof + static_cast<size_t>(i) * 24 + 6 * l;
+  st.p = V3{r[0], r[1], r[2]};
+  st.qx = r[3]; st.qy = r[4]; st.qz = r[5]; st.qw = r[6];
+  const G3 R = quat_to_rot(st.qx, st.qy, st.qz, st.qw);
+  st.v = mulT(R, V3{r[7], r[8], r[9]});
+  st.w = mulT(R, V3{r[10], r[11], r[12]});
+  float tau[3], ff[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    st.q[k] = d[2 * k];
+    st.qd[k] = d[2 * k + 1];
+    tau[k] = torques[static_cast<size_t>(i) * 12 + 3 * l + k];
+  }
+  physics_step_elim_leg(a, lp, kElimTab.k[l], st, tau, ff);
+  if (l == 0) leg_root(st, r);   // after every lane of the quad has read the root (one wavefront)
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    d[2 * k] = st.q[k];
+    d[2 * k + 1] = st.qd[k];
+    if (foot_force) foot_force[static_cast<size_t>(i) * 12 + 3 * l + k] = ff[k];
   }
 }
 
@@ -127,8 +169,12 @@ int spi_physics_step(const SpiSimArgs* sim, const float* params_dev, int ld, int
   if (n < 0 || ld < n || !params_dev || !root_dev || !dof_state_dev || !torques_dev)
     return rfail(SPI_ERR_INVALID_ARG, "spi_physics_step: bad sizes or null pointer");
   if (n == 0) return SPI_OK;
-  physics_step_kernel<<<(n + 255) / 256, 256, 0, stream>>>(*sim, params_dev, ld, n, root_dev, dof_state_dev,
-                                                          torques_dev, foot_force_dev);
+  if (n <= kLegStepMaxEnvs)
+    physics_step_leg_kernel<<<(n + 63) / 64, 256, 0, stream>>>(*sim, params_dev, ld, n, root_dev, dof_state_dev,
+                                                               torques_dev, foot_force_dev);
+  else
+    physics_step_kernel<<<(n + 255) / 256, 256, 0, stream>>>(*sim, params_dev, ld, n, root_dev, dof_state_dev,
+                                                            torques_dev, foot_force_dev);
   return launched();
 }
 
