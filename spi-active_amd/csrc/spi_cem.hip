@@ -70,16 +70,13 @@ __global__ void cem_sample_kernel(const float* __restrict__ mean, const float* _
   }
 }
 
-// cost_dev[c] = sum_s w[s] * cost_seg[s][c]: one thread per candidate, segments in a fixed
-// order, so the per-candidate cost (and the CEM ranking) is deterministic.  Built with strict
-// IEEE semantics so +inf (diverged) costs propagate; a segment of weight 0 is skipped (its
-// cost may be +inf).  The loads of eight segments are issued together (they are independent;
-// one at a time, a 256-candidate landscape waited on 64 dependent load latencies), the sum
-// keeps the segment order.
-__global__ void reduce_segments_kernel(const float* __restrict__ cs, const float* __restrict__ w, int n_seg,
-                                       int n_cand, float* __restrict__ out) {
-  int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= n_cand) return;
+// Cost of candidate c: sum_s w[s] * cost_seg[s][c], segments in a fixed order, so that the cost (and
+// the CEM ranking) is deterministic.  Built with strict IEEE semantics so +inf (diverged) costs
+// propagate; a segment of weight 0 is skipped (its cost may be +inf).  The loads of eight segments
+// are issued together (they are independent; one at a time, a 256-candidate landscape waited on 64
+// dependent load latencies), the sum keeps the segment order.
+__device__ __forceinline__ float weighted_cost(const float* __restrict__ cs, const float* __restrict__ w, int n_seg,
+                                               int n_cand, int c) {
   float acc = 0.0f;
   int s = 0;
   for (; s + 8 <= n_seg; s += 8) {
@@ -97,19 +94,109 @@ __global__ void reduce_segments_kernel(const float* __restrict__ cs, const float
     float ws = w[s];
     if (ws != 0.0f) acc += ws * cs[static_cast<size_t>(s) * n_cand + c];
   }
-  out[c] = acc;
+  return acc;
 }
 
+// cost_dev[c], one thread per candidate.
+__global__ void reduce_segments_kernel(const float* __restrict__ cs, const float* __restrict__ w, int n_seg,
+                                       int n_cand, float* __restrict__ out) {
+  int c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c < n_cand) out[c] = weighted_cost(cs, w, n_seg, n_cand, c);
+}
 
 constexpr int kCemThreads = 1024;
 
-// (cost, index) pairs sorted ascending in LDS (bitonic network, ties broken by index, NaN
-// treated as +inf), then per-parameter elite moments with wave reductions and the best-so-far.
-// Called by one whole workgroup of kCemThreads threads; keys must already hold the costs.
-__device__ void cem_sort_update(float* key, int* val, int n, int npow2, const float* __restrict__ theta, int ld,
-                                int n_param, int n_elite, float alpha, const float* __restrict__ min_std,
-                                float* __restrict__ mean, float* __restrict__ stdv, float* __restrict__ best,
-                                float* __restrict__ best_cost, int* __restrict__ elite_idx) {
+constexpr int kSelectMax = 1024;   // elites that the selection handles; more are sorted
+constexpr int kListMax = 2048;     // candidates up to the threshold (its ties included)
+
+// Order of the ranking as unsigned integers: ascending cost, NaN as +inf, -0 as 0.
+__device__ __forceinline__ unsigned order_bits(float c) {
+  unsigned u = c == c ? __float_as_uint(c) : 0x7f800000u;
+  if ((u << 1) == 0) u = 0;
+  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+
+// The n_elite lowest (cost, index) pairs in ascending order into val[0 .. n_elite), for n_elite <=
+// kSelectMax: the n_elite-th lowest cost by four 8-bit counting passes over the keys, then the
+// candidates up to it ranked against each other.  False (val undefined) if more than kListMax
+// candidates tie up to the threshold.  A sort of all 4096 pairs took 78 barriers of about a
+// microsecond each; this takes a dozen.  Called by a whole workgroup.
+__device__ bool select_elites(const float* key, int* val, unsigned long long* list, int n, int n_elite) {
+  __shared__ int hist[256];
+  __shared__ unsigned prefix_s;
+  __shared__ int want_s, count_s;
+  const int tid = threadIdx.x, lane = tid & 63;
+  unsigned prefix = 0;     // digits of the threshold so far
+  int want = n_elite;      // its rank among the keys that share them
+  for (int shift = 24; shift >= 0; shift -= 8) {
+    if (tid < 256) hist[tid] = 0;
+    __syncthreads();
+    for (int i0 = 0; i0 < n; i0 += kCemThreads) {
+      const int i = i0 + tid;
+      const unsigned u = i < n ? order_bits(key[i]) : 0u;
+      bool live = i < n && (shift == 24 || (u >> (shift + 8)) == prefix);
+      const unsigned d = (u >> shift) & 255u;
+      // costs of one population share their leading digits: the wave's commonest digits are
+      // counted by ballot, one LDS atomic for all their lanes
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        const unsigned long long any = __ballot(live);
+        if (any) {
+          const unsigned d0 = __shfl(d, __ffsll(any) - 1, 64);
+          const bool same = live && d == d0;
+          const unsigned long long m = __ballot(same);
+          if (lane == __ffsll(m) - 1) atomicAdd(&hist[d0], __popcll(m));
+          live = live && !same;
+        }
+      }
+      if (live) atomicAdd(&hist[d], 1);
+    }
+    __syncthreads();
+    if (tid < 64) {        // the digit whose cumulated count reaches `want`
+      int h[4], sum = 0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) { h[k] = hist[4 * lane + k]; sum += h[k]; }
+      int incl = sum;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const int o = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += o;
+      }
+      int below = incl - sum;
+      if (below < want && incl >= want) {
+        int k = 0;
+        while (below + h[k] < want) below += h[k++];
+        prefix_s = (prefix << 8) | static_cast<unsigned>(4 * lane + k);
+        want_s = want - below;
+      }
+      if (tid == 0) count_s = 0;
+    }
+    __syncthreads();
+    prefix = prefix_s;
+    want = want_s;
+  }
+  for (int i = tid; i < n; i += kCemThreads) {
+    const unsigned u = order_bits(key[i]);
+    if (u <= prefix) {
+      const int at = atomicAdd(&count_s, 1);
+      if (at < kListMax) list[at] = (static_cast<unsigned long long>(u) << 32) | static_cast<unsigned>(i);
+    }
+  }
+  __syncthreads();
+  const int m = count_s;
+  if (m > kListMax) return false;
+  for (int e = tid; e < m; e += kCemThreads) {
+    const unsigned long long x = list[e];
+    int rank = 0;
+    for (int o = 0; o < m; ++o) rank += list[o] < x;   // distinct: the index is part of the value
+    if (rank < n_elite) val[rank] = static_cast<int>(x & 0xffffffffu);
+  }
+  __syncthreads();
+  return true;
+}
+
+// All (cost, index) pairs sorted ascending in LDS (bitonic network, ties broken by index).
+__device__ void sort_all(float* key, int* val, int n, int npow2) {
   const int tid = threadIdx.x;
   for (int i = tid; i < npow2; i += kCemThreads) {
     float c = i < n ? key[i] : INFINITY;
@@ -132,21 +219,67 @@ __device__ void cem_sort_update(float* key, int* val, int n, int npow2, const fl
       __syncthreads();
     }
   }
+}
+
+constexpr int kEliteRegs = kSelectMax / 64;
+
+// Elites in ascending order of (cost, index), NaN treated as +inf (selected where they are few,
+// else by sorting all), then per-parameter elite moments with wave reductions and the best-so-far.
+// Called by one whole workgroup of kCemThreads threads; keys must already hold the costs.  One
+// workgroup's latency is the time: 4096 samples, 410 elites, 25 parameters 77 -> 40 us.
+__device__ void cem_sort_update(float* key, int* val, unsigned long long* list, int n, int npow2,
+                                const float* __restrict__ theta, int ld, int n_param, int n_elite, float alpha,
+                                const float* __restrict__ min_std, float* __restrict__ mean, float* __restrict__ stdv,
+                                float* __restrict__ best, float* __restrict__ best_cost, int* __restrict__ elite_idx) {
+  const int tid = threadIdx.x;
+  __shared__ float best_key;
+  if (n_elite <= kSelectMax && select_elites(key, val, list, n, n_elite)) {
+    if (tid == 0) best_key = key[val[0]] == key[val[0]] ? key[val[0]] : INFINITY;
+  } else {
+    __syncthreads();
+    sort_all(key, val, n, npow2);
+    if (tid == 0) best_key = key[0];
+  }
+  __syncthreads();
   if (elite_idx)
     for (int e = tid; e < n_elite; e += kCemThreads) elite_idx[e] = val[e];
   // one wave per parameter: lanes stride over the elites, then a fixed butterfly
   const int wave = tid / 64, lane = tid % 64, n_waves = kCemThreads / 64;
   for (int p = wave; p < n_param; p += n_waves) {
     const float* th = theta + static_cast<size_t>(p) * ld;
+    // both passes over the same values, in the same order: gathered once, all loads in flight,
+    // where a lane's share fits its registers
+    float x[kEliteRegs];
+    const bool held = n_elite <= kSelectMax;
+    if (held) {
+#pragma unroll
+      for (int k = 0; k < kEliteRegs; ++k)
+        if (lane + 64 * k < n_elite) x[k] = th[val[lane + 64 * k]];
+    }
     float s = 0.0f;
-    for (int e = lane; e < n_elite; e += 64) s += th[val[e]];
+    if (held) {
+#pragma unroll
+      for (int k = 0; k < kEliteRegs; ++k)
+        if (lane + 64 * k < n_elite) s += x[k];
+    } else {
+      for (int e = lane; e < n_elite; e += 64) s += th[val[e]];
+    }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
     const float m = s / static_cast<float>(n_elite);
     float v = 0.0f;
-    for (int e = lane; e < n_elite; e += 64) {
-      float d = th[val[e]] - m;
-      v += d * d;
+    if (held) {
+#pragma unroll
+      for (int k = 0; k < kEliteRegs; ++k)
+        if (lane + 64 * k < n_elite) {
+          float d = x[k] - m;
+          v += d * d;
+        }
+    } else {
+      for (int e = lane; e < n_elite; e += 64) {
+        float d = th[val[e]] - m;
+        v += d * d;
+      }
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
@@ -160,11 +293,11 @@ __device__ void cem_sort_update(float* key, int* val, int n, int npow2, const fl
   }
   // best sample so far: replaced only when this iteration's best strictly improves it
   __shared__ int improved;
-  if (tid == 0) improved = key[0] < best_cost[0];
+  if (tid == 0) improved = best_key < best_cost[0];
   __syncthreads();
   if (improved) {
     for (int p = tid; p < n_param; p += kCemThreads) best[p] = theta[static_cast<size_t>(p) * ld + val[0]];
-    if (tid == 0) best_cost[0] = key[0];
+    if (tid == 0) best_cost[0] = best_key;
   }
   __syncthreads();
 }
@@ -175,9 +308,10 @@ __global__ __launch_bounds__(kCemThreads) void cem_update_kernel(
     float* __restrict__ best, float* __restrict__ best_cost, int* __restrict__ elite_idx, int npow2) {
   __shared__ float key[SPI_MAX_CEM_SAMPLES];
   __shared__ int val[SPI_MAX_CEM_SAMPLES];
+  __shared__ unsigned long long list[kListMax];
   for (int i = threadIdx.x; i < n; i += kCemThreads) key[i] = cost[i];
   __syncthreads();
-  cem_sort_update(key, val, n, npow2, theta, ld, n_param, n_elite, alpha, min_std, mean, stdv, best, best_cost,
+  cem_sort_update(key, val, list, n, npow2, theta, ld, n_param, n_elite, alpha, min_std, mean, stdv, best, best_cost,
                   elite_idx);
 }
 
@@ -206,21 +340,18 @@ __global__ void cem_sample_batch_kernel(const SpiBatchProblem* __restrict__ prob
 __global__ __launch_bounds__(kCemThreads) void cem_update_batch_kernel(SpiBatchProblem* __restrict__ probs) {
   __shared__ float key[SPI_MAX_CEM_SAMPLES];
   __shared__ int val[SPI_MAX_CEM_SAMPLES];
+  __shared__ unsigned long long list[kListMax];
   SpiBatchProblem& P = probs[blockIdx.x];
   const int n = P.n_samples;
   for (int c = threadIdx.x; c < n; c += kCemThreads) {
-    float acc = 0.0f;
-    for (int s = 0; s < P.n_seg; ++s) {
-      float ws = P.seg_weight[s];
-      if (ws != 0.0f) acc += ws * P.cost_seg[static_cast<size_t>(s) * n + c];
-    }
+    const float acc = weighted_cost(P.cost_seg, P.seg_weight, P.n_seg, n, c);
     P.cost_out[c] = acc;
     key[c] = acc;
   }
   __syncthreads();
   int npow2 = 2;
   while (npow2 < n) npow2 <<= 1;
-  cem_sort_update(key, val, n, npow2, P.theta, n, SPI_P_COUNT, P.n_elite, P.alpha, P.min_std, P.mean, P.std,
+  cem_sort_update(key, val, list, n, npow2, P.theta, n, SPI_P_COUNT, P.n_elite, P.alpha, P.min_std, P.mean, P.std,
                   P.best, P.best_cost, nullptr);
   if (threadIdx.x == 0) P.iteration = P.iteration + 1u;
 }
