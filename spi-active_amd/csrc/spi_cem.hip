@@ -108,6 +108,7 @@ constexpr int kCemThreads = 1024;
 
 constexpr int kSelectMax = 1024;   // elites that the selection handles; more are sorted
 constexpr int kListMax = 2048;     // candidates up to the threshold (its ties included)
+static_assert(kSelectMax <= kListMax && 2 * kListMax <= SPI_MAX_CEM_SAMPLES, "val holds the elites and the ranks");
 
 // Order of the ranking as unsigned integers: ascending cost, NaN as +inf, -0 as 0.
 __device__ __forceinline__ unsigned order_bits(float c) {
@@ -185,12 +186,22 @@ __device__ bool select_elites(const float* key, int* val, unsigned long long* li
   __syncthreads();
   const int m = count_s;
   if (m > kListMax) return false;
-  for (int e = tid; e < m; e += kCemThreads) {
+  // rank of each against all, the comparisons of one candidate shared by as many threads as there are
+  int* rank = val + kListMax;
+  for (int e = tid; e < m; e += kCemThreads) rank[e] = 0;
+  __syncthreads();
+  const int parts = m < kCemThreads ? kCemThreads / m : 1;
+  for (int t = tid; t < m * parts; t += kCemThreads) {
+    const int e = t % m;
     const unsigned long long x = list[e];
-    int rank = 0;
-    for (int o = 0; o < m; ++o) rank += list[o] < x;   // distinct: the index is part of the value
-    if (rank < n_elite) val[rank] = static_cast<int>(x & 0xffffffffu);
+    int r = 0;
+#pragma unroll 8
+    for (int o = t / m; o < m; o += parts) r += list[o] < x;   // distinct: the index is part of the value
+    if (parts > 1) atomicAdd(&rank[e], r); else rank[e] = r;
   }
+  __syncthreads();
+  for (int e = tid; e < m; e += kCemThreads)
+    if (rank[e] < n_elite) val[rank[e]] = static_cast<int>(list[e] & 0xffffffffu);
   __syncthreads();
   return true;
 }
@@ -226,7 +237,7 @@ constexpr int kEliteRegs = kSelectMax / 64;
 // Elites in ascending order of (cost, index), NaN treated as +inf (selected where they are few,
 // else by sorting all), then per-parameter elite moments with wave reductions and the best-so-far.
 // Called by one whole workgroup of kCemThreads threads; keys must already hold the costs.  One
-// workgroup's latency is the time: 4096 samples, 410 elites, 25 parameters 77 -> 40 us.
+// workgroup's latency is the time: 4096 samples, 410 elites, 25 parameters 77 -> 32 us.
 __device__ void cem_sort_update(float* key, int* val, unsigned long long* list, int n, int npow2,
                                 const float* __restrict__ theta, int ld, int n_param, int n_elite, float alpha,
                                 const float* __restrict__ min_std, float* __restrict__ mean, float* __restrict__ stdv,
