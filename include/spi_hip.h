@@ -388,6 +388,17 @@ int spi_pack_windows(const float* states_dev, const float* actions_dev, int n_st
  * is read.  The device side of the loop over recorded files in scripts/eval.py:101-171. */
 int spi_pack_windows_rows(const float* states_dev, const float* actions_dev, int n_rows, const int* rows_dev,
                           int n_windows, int horizon, float* segments_dev, hipStream_t stream);
+/* spi_pack_windows over every window of n_traj trajectories held back to back, each longer than
+ * horizon: trajectory i starts at row first_dev[i] (first_dev[0] == 0), n_windows == n_rows -
+ * n_traj * horizon.  No row table: window w of trajectory i starts at row w + i * horizon. */
+int spi_pack_windows_store(const float* states_dev, const float* actions_dev, int n_rows, const int* first_dev,
+                           int n_traj, int n_windows, int horizon, float* segments_dev, hipStream_t stream);
+/* Host side of the same loop: for the counts[k] windows of chosen trajectory traj[k] (first row
+ * first[k], gains kp[k], kd[k]), k < n, in order, the window's trajectory, start step, gains,
+ * row (rows may be null) and whether it is its trajectory's last. Host pointers. */
+int spi_window_index(int n, const int* traj, const int* counts, const int* first, const float* kp, const float* kd,
+                     unsigned char* ends_out, int* traj_out, int* start_out, float* kp_out, float* kd_out,
+                     int* rows_out);
 
 /* Tracking cost and its exact gradient with respect to all 25 parameter rows for every
  * (segment, candidate) pair, by reverse mode (adjoint) with checkpoints every

@@ -59,11 +59,13 @@ class SegmentStore:
         self.device = torch.device(device)
         self.trajectories: List[Trajectory] = []
         self._joined = None           # (states [R, 37], actions [R, 12], first row of each trajectory)
+        self._first_dev = None        # the first rows on the device
 
     def _joined_buffers(self):
         """All trajectories back to back in one device buffer (rebuilt after an add)."""
         if self._joined is None or len(self._joined[2]) != len(self.trajectories):
             starts = np.cumsum([0] + [tr.n_steps for tr in self.trajectories])[:-1]
+            self._first_dev = torch.from_numpy(np.minimum(starts, 2 ** 31 - 1).astype(np.int32)).to(self.device)
             self._joined = (torch.cat([tr.states for tr in self.trajectories]),
                             torch.cat([tr.actions for tr in self.trajectories]), starts)
         return self._joined
@@ -95,26 +97,31 @@ class SegmentStore:
         if n == 0:
             raise ValueError("no trajectory is longer than the horizon")
         out = torch.empty((n, segment_stride(horizon)), dtype=torch.float32, device=self.device)
-        ends = np.zeros(n, bool)
-        src, start, kp, kd = (np.zeros(n, np.int32), np.zeros(n, np.int32), np.zeros(n, np.float32),
-                              np.zeros(n, np.float32))
         states, actions, first = self._joined_buffers()
         if states.shape[0] >= 2 ** 31:
             raise ValueError("the store holds more than 2^31 - 1 trajectory rows")
-        rows = np.zeros(n, np.int32)
-        o = 0
-        for i, c in zip(which, counts):
-            if c == 0:
-                continue
-            tr = self.trajectories[i]
-            ends[o + c - 1] = True
-            src[o:o + c], start[o:o + c] = i, np.arange(c)
-            rows[o:o + c] = first[i] + np.arange(c)
-            kp[o:o + c], kd[o:o + c] = tr.kp, tr.kd
-            o += c
+        # every window of every trajectory: the kernel finds the rows itself; a choice of
+        # trajectories, or one no longer than the horizon, goes by a row table
+        whole = which == list(range(len(self.trajectories))) and min(counts) > 0
+        i32, f32 = np.int32, np.float32
+        ends, src, start = np.empty(n, bool), np.empty(n, i32), np.empty(n, i32)
+        kp, kd, rows = np.empty(n, f32), np.empty(n, f32), None if whole else np.empty(n, i32)
+        traj = np.asarray(which, i32)
+        table = (traj, np.asarray(counts, i32), first[traj].astype(i32),
+                 np.asarray([self.trajectories[i].kp for i in which], f32),
+                 np.asarray([self.trajectories[i].kd for i in which], f32))
+        L = _lib.lib()
+        if whole:
+            rc = L.spi_pack_windows_store(_lib.ptr(states), _lib.ptr(actions), states.shape[0],
+                                          _lib.ptr(self._first_dev, torch.int32), len(which), n, horizon, _lib.ptr(out),
+                                          _lib.stream())
+            _lib.check(rc, "spi_pack_windows_store")
+        L.spi_window_index(len(which), *[a.ctypes.data for a in table], ends.ctypes.data, src.ctypes.data,
+                           start.ctypes.data, kp.ctypes.data, kd.ctypes.data, None if whole else rows.ctypes.data)
+        if whole:
+            return SegmentBatch(out, horizon, ends, src, start, kp, kd)
         rows_dev = torch.from_numpy(rows).to(self.device)
-        rc = _lib.lib().spi_pack_windows_rows(_lib.ptr(states), _lib.ptr(actions), states.shape[0],
-                                              _lib.ptr(rows_dev, torch.int32), n, horizon, _lib.ptr(out),
-                                              _lib.stream())
+        rc = L.spi_pack_windows_rows(_lib.ptr(states), _lib.ptr(actions), states.shape[0],
+                                     _lib.ptr(rows_dev, torch.int32), n, horizon, _lib.ptr(out), _lib.stream())
         _lib.check(rc, "spi_pack_windows_rows")
         return SegmentBatch(out, horizon, ends, src, start, kp, kd)

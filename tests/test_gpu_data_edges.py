@@ -1,0 +1,52 @@
+"""Window packing and command sequences where their kernels change path: groups across the end of
+a trajectory, trajectories of one window, records longer than the staging, trajectories no longer
+than the horizon; trials shorter and longer than a workgroup, odd command widths."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("lengths,horizon", [((65, 64, 200), 1), ((21, 22, 40, 85, 21), 20), ((150, 129, 300), 128),
+                                             ((400, 371), 320), ((30, 5, 90), 20), ((700,), 7)])
+def test_store_windows_equal_the_rows(gpu, lengths, horizon):
+    from spi_amd.store import SegmentStore
+    rng = np.random.default_rng(sum(lengths))
+    store, data = SegmentStore(), []
+    for i, T in enumerate(lengths):
+        s, a = rng.normal(size=(T, 37)).astype(np.float32), rng.normal(size=(T, 12)).astype(np.float32)
+        store.add_arrays(s, a, kp=20.0 + i, kd=0.5 + i)
+        data.append((s, a))
+    for which in (None, list(range(len(lengths)))[::-1]):
+        b = store.windows(horizon, which)
+        want, src, start, ends = [], [], [], []
+        for i in (range(len(lengths)) if which is None else which):
+            s, a = data[i]
+            for t in range(len(s) - horizon):
+                rec = np.concatenate([a[t:t + horizon], s[t + 1:t + horizon + 1]], 1).reshape(-1)
+                want.append(np.concatenate([s[t], rec]))
+                src.append(i)
+                start.append(t)
+                ends.append(t == len(s) - horizon - 1)
+        assert np.array_equal(b.segments.cpu().numpy(), np.stack(want))
+        assert np.array_equal(b.source, src) and np.array_equal(b.start, start) and np.array_equal(b.motion_ends, ends)
+        assert np.array_equal(b.kp, 20.0 + np.array(src)) and np.array_equal(b.kd, np.float32(0.5) + np.array(src))
+
+
+@pytest.mark.parametrize("mode", ["constant", "polynomial", "bezier"])
+@pytest.mark.parametrize("trials,steps,width", [(1, 38, 14), (33, 39, 13), (5, 51, 14), (1, 52, 13), (2100, 50, 13), (3, 250, 11)])
+def test_command_sequences_at_edges(gpu, mode, trials, steps, width):
+    import torch
+    import spio_commands as oc
+    from spi_amd.agents.commands import CommandGenerator
+    from test_commands_oracle import DEFAULT, IDX, RANGES
+    gen = CommandGenerator(RANGES[:width], DEFAULT[:width], IDX, mode, rollout_length=5.0, horizon_length=1.0,
+                           dt=1.0 / steps)
+    U, S = gen.n_updates, gen.steps
+    rng = np.random.default_rng(trials)
+    b = gen.param_bounds()
+    P = rng.uniform(b[:, 0], b[:, 1], size=(trials, b.shape[0])).astype(np.float32)
+    out = gen.generate(torch.from_numpy(P)).cpu().numpy()
+    for k in sorted({0, trials // 2, trials - 1}):
+        ref = oc.commands_from_params(P[k], mode, RANGES[:width], DEFAULT[:width], IDX, U, S)
+        assert np.abs(out[k] - ref).max() < 2e-6
