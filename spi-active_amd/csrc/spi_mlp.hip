@@ -1,12 +1,13 @@
 // Policy network inference (gfx950): the actor MLP of the locomotion policy (Linear layers with
 // ELU between them, spigym/agents/modules/modules.py:47-63; hidden sizes 512-256-128 from
-// config/algo/ppo.yaml) as FP32 MFMA (v_mfma_f32_32x32x2f32) tiles, one launch per layer with
-// bias and ELU in the epilogue.  linear_kernel: a workgroup of 4 wavefronts owns a 32-row x
-// 128-column output tile (many workgroups for small batches); rows of X and the weight rows are
-// staged through LDS in K chunks of 64 (even columns, then odd ones, 65 words per row, so the
-// operand reads of a wavefront hit 64 distinct banks).  linear_db_kernel: 128 x 128 (a 64 x 64
-// quadrant per wavefront, K chunks of 32 double-buffered in LDS) for batches of 8192 rows and
-// more.  Strict IEEE float32 (no fast-math).
+// config/algo/ppo.yaml), one launch per layer with bias and ELU in the epilogue.
+// linear_split_kernel: layers of at least 64 inputs and outputs, float32 products formed exactly
+// enough on the bf16 matrix pipe.  linear_kernel: the others and the fused last two layers, FP32
+// MFMA (v_mfma_f32_32x32x2f32); a workgroup of 4 wavefronts owns a 32-row x 128-column output
+// tile, rows of X and the weight rows staged through LDS in K chunks of 64 (even columns, then odd
+// ones, 65 words per row, so the operand reads of a wavefront hit 64 distinct banks).  Strict IEEE
+// float32 (no fast-math).
+// The actor (900 -> 512 -> 256 -> 128 -> 12): 2048 rows 63 -> 50 us, 16384 rows 222 -> 175 us.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -31,7 +32,6 @@ constexpr int kKc = 64;      // K chunk staged per pass
 constexpr int kPad = kKc + 1;
 constexpr int kMaxLayers = 8;
 constexpr int kMaxRingK = 1024;  // widest ring-gathered input
-constexpr int kBigM = 8192;      // batches from here on use linear_db_kernel (N >= 256)
 
 // LDS slot of tile element (row, k): the even columns of a row first, then the odd ones, so
 // the MFMA operand reads of a wavefront (lane -> row l % 32, column kk + l / 32) cover 64
@@ -87,7 +87,7 @@ __global__ __launch_bounds__(256 * kS) void linear_kernel(const float* __restric
   constexpr int kPs = kKs + 1;
   constexpr int kGroupFloats = (kRows + kCols) * kPs;
   static_assert(kS == 1 || (kS - 1) * 16 * 256 <= kS * kGroupFloats, "reduction buffer fits the tiles");
-  static_assert(kRows * (kCols + 1) + 2 * kRows * 32 <= kS * kGroupFloats, "a fused tail's tile fits the tiles");
+  static_assert(kRows * (kCols + 1) + 2 * kRows * 32 + 32 * (kCols + 1) <= (kFuse ? kS * kGroupFloats : 1 << 20), "a fused tail's tile fits the tiles");
   __shared__ float smem[kS * kGroupFloats];
   __shared__ int Kr[kSrc >= 2 ? kMaxRingK : 1];       // ring line of each input column
   const int m0 = blockIdx.x * kRows, n0 = blockIdx.y * kCols;
@@ -218,7 +218,15 @@ __global__ __launch_bounds__(256 * kS) void linear_kernel(const float* __restric
     // every thread of every group reaches both barriers; group 0 holds the finished tile
     constexpr int kHs = kCols + 1;
     float* h = smem;                                   // [32][kHs] after the reduction reads
+    float* part = h + kRows * kHs;                     // [2][32][32] partial sums of the last layer
+    // the last layer's weights, each read 32 times: from global memory the 64-deep chains waited
+    // on a load every 8 steps
+    float* w2s = part + 2 * kRows * 32;                // [N2][kHs]
     __syncthreads();
+    for (int u = threadIdx.x; u < N2 * N; u += blockDim.x) {
+      const int j = u / N;
+      w2s[j * kHs + (u - j * N)] = W2[u];
+    }
     if (grp == 0) {
       const int gn = wave * 32 + col;
       const float bias = gn < N ? b[gn] : 0.0f;
@@ -236,13 +244,12 @@ __global__ __launch_bounds__(256 * kS) void linear_kernel(const float* __restric
     __syncthreads();
     // every thread: partial sums over the two halves of the N inputs, (half, row, output) per
     // thread, then half 0 + half 1 + bias in that order
-    float* part = h + kRows * kHs;                     // [2][32][32]
     const int nh = (N + 1) / 2;
     for (int u = threadIdx.x; u < 2 * kRows * N2; u += blockDim.x) {
       const int q = u / (kRows * N2), rem = u - q * (kRows * N2), row = rem / N2, j = rem - row * N2;
       const int k0 = q * nh, k1 = min(N, k0 + nh);
       const float* hr = h + row * kHs;
-      const float* w2 = W2 + static_cast<size_t>(j) * N;
+      const float* w2 = w2s + j * kHs;
       float sum = 0.0f;
 #pragma unroll 8
       for (int k = k0; k < k1; ++k) sum = fmaf(hr[k], w2[k], sum);
@@ -278,36 +285,81 @@ int split_for(int M, int K, int N) {
   return tiles <= 128 ? 4 : 2;
 }
 
-// Large batches: a workgroup of 4 wavefronts owns a 128 x 128 output tile, each wavefront a
-// 64 x 64 quadrant (2 x 2 MFMA blocks, 4 accumulators), so every LDS operand read feeds two
-// MFMAs.  K is staged in chunks of 32 through two LDS buffers (rows of 32 floats + 2 of padding,
-// 68 KB in all, so two workgroups share a CU): while the wavefronts multiply chunk c out of one
-// buffer, chunk c + 1 goes from registers into the other and chunk c + 2 is fetched into
-// registers, with one barrier per chunk.  In MFMA step s of a chunk the lanes of half h supply
-// column 16 h + s of both operands, read as float2 pairs (s, s + 1); in the last, ragged chunk
-// only the steps that reach a column below K run.  kSrc 0: X row-major (rows 16-byte aligned,
-// K % 4 == 0), float4 loads along the rows; 1: X gathered from a RingSrc whose lines are
-// 16-byte aligned with ld % 4 == 0, float4 loads of 4 rows of one column (lane l of a wavefront
-// covers rows 4 (l % 8) .. + 3 and column l / 8, so that the 64 lanes' LDS stores of one row
-// offset fall in 64 distinct banks); 2: any RingSrc, one row's four consecutive columns per
-// thread in scalar loads.  The accumulation order over K depends only on the tile layout, not
-// on the source, so the dense and the ring input give the same bits.
-constexpr int kDbRows = 128, kDbCols = 128, kDbK = 32, kDbStride = kDbK + 2, kDbTile = 128 * kDbStride;
-template <bool kElu, int kSrc>
-__global__ __launch_bounds__(256) void linear_db_kernel(const float* __restrict__ X, int ldx, RingSrc rs, int M,
-                                                        int K, const float* __restrict__ W,
-                                                        const float* __restrict__ b, int N, float* __restrict__ Y,
-                                                        int ldy) {
-  __shared__ __attribute__((aligned(16))) float lds[2 * 2 * kDbTile];   // [buffer][A | W][row][34]
+// float32 products on the bf16 matrix pipe.  A float is exactly the sum of three bf16 values (its
+// 24 significant bits in 8 + 8 + 8, each part truncated), so a product is nine bf16 products;
+// the six largest are kept (the dropped ones are below 2^-22 of it) and accumulated in float32:
+// six v_mfma_f32_32x32x16_bf16 of 32 cycles replace eight v_mfma_f32_32x32x2_f32 of 64.  The
+// leading products and the five small ones have an accumulator each, so the leading one adds 57
+// times where the float32 pipe added 450 times for 900 inputs: the error of the whole actor against 64
+// bits fell from 3.3e-7 .. 6.4e-7 to 2.5e-7 .. 3.5e-7 (batches of 16 .. 16384 rows).
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+struct Split4 { uint2 p[3]; };      // the three parts of four consecutive inputs
+__device__ __forceinline__ Split4 split4(const float* x) {
+  unsigned u[3][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    u[0][i] = __float_as_uint(x[i]);
+    const float r = x[i] - __uint_as_float(u[0][i] & 0xffff0000u);
+    u[1][i] = __float_as_uint(r);
+    u[2][i] = __float_as_uint(r - __uint_as_float(u[1][i] & 0xffff0000u));
+  }
+  Split4 s;
+#pragma unroll
+  for (int q = 0; q < 3; ++q)   // the high halves of two words
+    s.p[q] = make_uint2(__builtin_amdgcn_perm(u[q][1], u[q][0], 0x07060302u),
+                        __builtin_amdgcn_perm(u[q][3], u[q][2], 0x07060302u));
+  return s;
+}
+
+// Tile of a workgroup: ids go round-robin over the 8 XCDs, and all column tiles of a row tile go to
+// one XCD one after the other, so that X is read from memory once and then from that XCD's L2.
+__device__ __forceinline__ void tile_of(int id, int n_tiles, int n_col, int* row, int* col) {
+  const int full = (n_tiles / n_col) / 8 * 8 * n_col;   // tiles of whole groups of 8 row tiles
+  if (id < full) {
+    const int j = id >> 3;
+    *row = j / n_col * 8 + (id & 7);
+    *col = j % n_col;
+  } else {
+    *row = id / n_col;
+    *col = id % n_col;
+  }
+}
+
+// linear_kernel's layer on the split products: 4 wavefronts own a 64 x 64 kN output tile, each a
+// quarter of 32 x 32 kN.  K goes in chunks of 32 through two LDS buffers: while chunk c is
+// multiplied, chunk c + 1 is split into the other buffer and chunks c + 2 and c + 3 are in flight.
+// LDS rows are four 16-byte units of 8 columns, unit u of row r at u ^ (r / 2) % 4: the 16-byte
+// operand reads of 8 rows and the 8-byte stores of a row's columns each cover the banks once.
+// Lane l supplies row l % 32 and columns 8 (l / 32) .. + 7 of both operands.
+// A wavefront issues 12 kN MFMAs (32 cycles each) and splits 8 (1 + kN) values (5.5 vector
+// instructions of 4 cycles each) per chunk, and the two do not overlap on a SIMD: kN = 2 halves
+// the splitting per product where the tiles still fill the chip.  kG groups of 4 wavefronts take
+// alternate chunks and add up in group order at the end: for batches of one tile per CU, whose
+// wavefronts would sit alone on their SIMDs.
+// kSrc 0: X row-major; 1: X gathered from a RingSrc in blocks of 2 rows x 4 columns, float2 along
+// the rows (lines 8-byte aligned, ld even); 2: the same blocks in scalar loads.  The accumulation
+// order does not depend on the source: dense and ring input give the same bits.
+// A result that is not finite (an infinite or NaN input has no finite parts) is formed again from
+// float32 products.
+constexpr int kSpTile = 64, kSpK = 32;
+constexpr int kSpGroupTiles = 256, kSpWideTiles = 1024;   // tiles of 64 x 64
+template <bool kElu, int kSrc, int kN, int kG>
+__global__ __launch_bounds__(256 * kG, 2) void linear_split_kernel(const float* __restrict__ X, int ldx, RingSrc rs,
+                                                                   int M, int K, const float* __restrict__ W,
+                                                                   const float* __restrict__ b, int N,
+                                                                   float* __restrict__ Y, int ldy) {
+  constexpr int kTc = kSpTile * kN, kRowsLds = kSpTile + kTc, kWPer = 2 * kN;
+  __shared__ uint4 lds[kG][2][3][kRowsLds * 4];        // [group][buffer][part][X rows, W rows][unit]
   constexpr bool kRing = kSrc != 0;
   __shared__ int Kr[kRing ? kMaxRingK : 1];
-  const int m0 = blockIdx.x * kDbRows, n0 = blockIdx.y * kDbCols;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  int rb, cb;
+  tile_of(blockIdx.x, gridDim.x, (N + kTc - 1) / kTc, &rb, &cb);
+  const int m0 = rb * kSpTile, n0 = cb * kTc;
+  const int grp = threadIdx.x >> 8, tid = threadIdx.x & 255, wave = tid >> 6, lane = tid & 63;
   const int col = lane & 31, half = lane >> 5;
-  const int wr = (wave >> 1) * 64, wc = (wave & 1) * 64;   // this wavefront's quadrant
-  const bool live = n0 + wc < N;                            // uniform per wavefront
+  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32 * kN;
   if (kRing) {
-    for (int k = tid; k < K; k += 256) {
+    for (int k = threadIdx.x; k < K; k += 256 * kG) {
       const int2 km = rs.kmap[k];
       const int back = min(max(km.x, 0), rs.n_slots - 1);
       const int slot = rs.head >= back ? rs.head - back : rs.head - back + rs.n_slots;
@@ -315,128 +367,153 @@ __global__ __launch_bounds__(256) void linear_db_kernel(const float* __restrict_
     }
     __syncthreads();
   }
-  floatx16 acc[2][2];
+  const int sr = tid >> 3, sc = (tid & 7) * 4;         // row-major: rows sr + 32 i, columns sc .. + 3
+  const int gr = (tid & 31) * 2, gc = (tid >> 5) * 4;  // ring: rows gr, gr + 1, columns gc .. + 3
+  // rows past the matrix read its last ones (their results are not stored)
+  const float* xsrc[2];
+  const float* wsrc[kWPer];
 #pragma unroll
-  for (int p = 0; p < 2; ++p)
+  for (int i = 0; i < 2; ++i)
+    xsrc[i] = kRing ? nullptr : X + static_cast<size_t>(min(m0 + sr + 32 * i, M - 1)) * ldx + sc;
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
+  for (int i = 0; i < kWPer; ++i) wsrc[i] = W + static_cast<size_t>(min(n0 + sr + 32 * i, N - 1)) * K + sc;
+  const int gq = min(m0 + gr, (M - 1) & ~1);           // rows up to M rounded to 2 exist in every line
+  struct Chunk { float x[2][4], w[kWPer][4]; };
+  auto load4 = [](float* o, const float* p, bool in) {
+    float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (in) v = *reinterpret_cast<const float4*>(p);
+    o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
+  };
+  auto fetch_at = [&](Chunk& o, int k0, bool whole) {   // whole: no column at or past K
+    const bool in = whole || k0 + sc < K;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[p][q][r] = 0.0f;
-  // W (and dense X) staging: thread -> rows (tid >> 3) + 32 i, columns 4 (tid & 7) .. + 3
-  const int sr = tid >> 3, sc = (tid & 7) * 4;
-  // float4 ring staging: thread -> rows 32 wave + 4 (lane % 8) .. + 3, columns lane / 8 + 8 i
-  const int fr = 32 * wave + 4 * (lane & 7), fk = lane >> 3;
-  // scalar ring staging: thread -> row tid & 127, column quads (tid >> 7) + 2 i
-  const int gr = tid & 127, gq = tid >> 7;
-  float4 ra[4], rw[4];
-  auto fetch = [&](int k0) {
+    for (int i = 0; i < kWPer; ++i) load4(o.w[i], wsrc[i] + k0, in);
+    if (!kRing) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (kSrc == 1) {
-        // rows up to M rounded to 4 exist in every line (ld >= that); rows >= M read as 0
-        const int gm = m0 + fr, k = k0 + fk + 8 * i;
-        float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (gm < M && k < K) v = *reinterpret_cast<const float4*>(rs.ring + static_cast<size_t>(Kr[k]) * rs.ld + gm);
-        ra[i].x = fminf(fmaxf(v.x, -rs.clip), rs.clip);
-        ra[i].y = gm + 1 < M ? fminf(fmaxf(v.y, -rs.clip), rs.clip) : 0.0f;
-        ra[i].z = gm + 2 < M ? fminf(fmaxf(v.z, -rs.clip), rs.clip) : 0.0f;
-        ra[i].w = gm + 3 < M ? fminf(fmaxf(v.w, -rs.clip), rs.clip) : 0.0f;
-      } else if (kSrc == 2) {
-        const int gm = m0 + gr, kq = k0 + 4 * (gq + 2 * i);
-        float v[4];
+      for (int i = 0; i < 2; ++i) load4(o.x[i], xsrc[i] + k0, in);
+    } else {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int k = kq + e;
-          v[e] = 0.0f;
-          if (gm < M && k < K)
-            v[e] = fminf(fmaxf(rs.ring[static_cast<size_t>(Kr[k]) * rs.ld + gm], -rs.clip), rs.clip);
+      for (int e = 0; e < 4; ++e) {
+        const int k = k0 + gc + e;
+        float2 q = make_float2(0.0f, 0.0f);
+        if (whole || k < K) {
+          const float* line = rs.ring + static_cast<size_t>(Kr[k]) * rs.ld;
+          if (kSrc == 1) q = *reinterpret_cast<const float2*>(line + gq);
+          else q = make_float2(line[min(m0 + gr, M - 1)], line[min(m0 + gr + 1, M - 1)]);
         }
-        ra[i] = make_float4(v[0], v[1], v[2], v[3]);
-      } else {
-        const int gm = m0 + sr + 32 * i, gk = k0 + sc;
-        ra[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (gm < M && gk < K) ra[i] = *reinterpret_cast<const float4*>(X + static_cast<size_t>(gm) * ldx + gk);
+        o.x[0][e] = q.x;
+        o.x[1][e] = q.y;
       }
-      const int gn = n0 + sr + 32 * i, gk = k0 + sc;
-      rw[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      if (gn < N && gk < K) rw[i] = *reinterpret_cast<const float4*>(W + static_cast<size_t>(gn) * K + gk);
     }
   };
-  auto stage = [&](int buf) {
-    float* A = lds + buf * 2 * kDbTile;
-    float* B = A + kDbTile;
+  auto fetch = [&](Chunk& o, int c) {                   // chunk c of this group
+    const int k0 = (c * kG + grp) * kSpK;
+    if (k0 + kSpK <= K) fetch_at(o, k0, true);
+    else fetch_at(o, k0, false);
+  };
+  auto put = [&](const float* v, int buf, int row, int c) {
+    const Split4 s = split4(v);
+    const int unit = row * 4 + ((c >> 3) ^ ((row >> 1) & 3));
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (kSrc == 1) {
-        float* pa = A + fr * kDbStride + fk + 8 * i;
-        pa[0] = ra[i].x;
-        pa[kDbStride] = ra[i].y;
-        pa[2 * kDbStride] = ra[i].z;
-        pa[3 * kDbStride] = ra[i].w;
-      } else {
-        float2* pa = reinterpret_cast<float2*>(kSrc == 2 ? A + gr * kDbStride + 4 * (gq + 2 * i)
-                                                         : A + (sr + 32 * i) * kDbStride + sc);
-        pa[0] = make_float2(ra[i].x, ra[i].y);
-        pa[1] = make_float2(ra[i].z, ra[i].w);
-      }
-      float2* pb = reinterpret_cast<float2*>(B + (sr + 32 * i) * kDbStride + sc);
-      pb[0] = make_float2(rw[i].x, rw[i].y);
-      pb[1] = make_float2(rw[i].z, rw[i].w);
-    }
+    for (int q = 0; q < 3; ++q) reinterpret_cast<uint2*>(&lds[grp][buf][q][unit])[(c >> 2) & 1] = s.p[q];
   };
-  auto compute = [&](int buf, int npair) {
-    const float* A = lds + buf * 2 * kDbTile;
-    const float* ap = A + (wr + col) * kDbStride + 16 * half;
-    const float* bp = A + kDbTile + (wc + col) * kDbStride + 16 * half;
+  auto stage = [&](Chunk& o, int buf) {
 #pragma unroll
-    for (int jp = 0; jp < kDbK / 4; ++jp) {          // steps s = 2 jp, 2 jp + 1
-      if (jp < npair) {
-        const float2 a0 = *reinterpret_cast<const float2*>(ap + 2 * jp);
-        const float2 a1 = *reinterpret_cast<const float2*>(ap + 32 * kDbStride + 2 * jp);
-        const float2 b0 = *reinterpret_cast<const float2*>(bp + 2 * jp);
-        const float2 b1 = *reinterpret_cast<const float2*>(bp + 32 * kDbStride + 2 * jp);
-        acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.x, b0.x, acc[0][0], 0, 0, 0);
-        acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.x, b1.x, acc[0][1], 0, 0, 0);
-        acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.x, b0.x, acc[1][0], 0, 0, 0);
-        acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.x, b1.x, acc[1][1], 0, 0, 0);
-        acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.y, b0.y, acc[0][0], 0, 0, 0);
-        acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.y, b1.y, acc[0][1], 0, 0, 0);
-        acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.y, b0.y, acc[1][0], 0, 0, 0);
-        acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.y, b1.y, acc[1][1], 0, 0, 0);
+    for (int i = 0; i < 2; ++i) {
+      if (kRing) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o.x[i][e] = fminf(fmaxf(o.x[i][e], -rs.clip), rs.clip);
+        put(o.x[i], buf, gr + i, gc);
+      } else {
+        put(o.x[i], buf, sr + 32 * i, sc);
       }
     }
+#pragma unroll
+    for (int i = 0; i < kWPer; ++i) put(o.w[i], buf, kSpTile + sr + 32 * i, sc);
   };
-  const int nch = (K + kDbK - 1) / kDbK;
-  fetch(0);
-  stage(0);
-  if (nch > 1) fetch(kDbK);
+  floatx16 hi[kN], lo[kN];
+#pragma unroll
+  for (int n = 0; n < kN; ++n)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) hi[n][r] = lo[n][r] = 0.0f;
+  auto operand = [&](int buf, int q, int row, int ks) {
+    return *reinterpret_cast<const bf16x8*>(&lds[grp][buf][q][row * 4 + ((2 * ks + half) ^ ((row >> 1) & 3))]);
+  };
+  auto compute = [&](int buf) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      bf16x8 x[3], w[kN][3];
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        x[q] = operand(buf, q, wr + col, ks);
+#pragma unroll
+        for (int n = 0; n < kN; ++n) w[n][q] = operand(buf, q, kSpTile + wc + 32 * n + col, ks);
+      }
+#define SPI_MM(A, P, Q)                                                                                  \
+  _Pragma("unroll") for (int n = 0; n < kN; ++n)                                                         \
+      A[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[P], w[n][Q], A[n], 0, 0, 0);
+      SPI_MM(lo, 2, 0)
+      SPI_MM(hi, 0, 0)
+      SPI_MM(lo, 0, 2)
+      SPI_MM(lo, 1, 1)
+      SPI_MM(lo, 1, 0)
+      SPI_MM(lo, 0, 1)
+#undef SPI_MM
+    }
+  };
+  const int nch = (K + kSpK * kG - 1) / (kSpK * kG);    // per group; chunks past K are zeros
+  Chunk even, odd;
+  fetch(even, 0);
+  fetch(odd, 1);
+  stage(even, 0);
+  fetch(even, 2);
   __syncthreads();
-  for (int c = 0; c < nch; ++c) {
-    // columns 16 + s of half 1 lie past K whenever column s does
-    const int klen = min(kDbK, K - c * kDbK);
-    const int npair = klen >= kDbK / 2 ? kDbK / 4 : (klen + 1) / 2;
-    if (live) compute(c & 1, npair);
-    if (c + 1 < nch) stage((c + 1) & 1);
-    if (c + 2 < nch) fetch((c + 2) * kDbK);
+  for (int c = 0; c < nch; c += 2) {
+    compute(0);
+    stage(odd, 1);
+    fetch(odd, c + 3);
+    __syncthreads();
+    if (c + 1 < nch) compute(1);
+    stage(even, 0);
+    fetch(even, c + 4);
     __syncthreads();
   }
-  if (!live) return;
+  if (kG > 1) {                                        // the loop ended on a barrier: the tiles are free
+    static_assert((kG - 1) * kN * 16 * 256 * 4 <= sizeof(lds), "the partial sums fit the tiles");
+    float* red = reinterpret_cast<float*>(lds);
+    if (grp > 0) {
 #pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const int gn = n0 + wc + 32 * q + col;
+      for (int n = 0; n < kN; ++n)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) red[(((grp - 1) * kN + n) * 16 + r) * 256 + tid] = hi[n][r] + lo[n][r];
+    }
+    __syncthreads();
+    if (grp > 0) return;
+  }
+#pragma unroll
+  for (int n = 0; n < kN; ++n) {
+    const int gn = n0 + wc + 32 * n + col;
     if (gn >= N) continue;
     const float bias = b[gn];
 #pragma unroll
-    for (int p = 0; p < 2; ++p)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int gm = m0 + wr + 32 * p + 8 * (r >> 2) + 4 * half + (r & 3);
-        if (gm < M) {
-          float v = acc[p][q][r] + bias;
-          if (kElu) v = v > 0.0f ? v : expm1f(v);
-          Y[static_cast<size_t>(gm) * ldy + gn] = v;
+    for (int r = 0; r < 16; ++r) {
+      const int gm = m0 + wr + 8 * (r >> 2) + 4 * half + (r & 3);
+      if (gm < M) {
+        float y = hi[n][r] + lo[n][r];
+        for (int g = 1; g < kG; ++g) y += reinterpret_cast<const float*>(lds)[(((g - 1) * kN + n) * 16 + r) * 256 + tid];
+        if (!isfinite(y)) {
+          y = 0.0f;
+          for (int k = 0; k < K; ++k) {
+            const float x = kRing ? fminf(fmaxf(rs.ring[static_cast<size_t>(Kr[k]) * rs.ld + gm], -rs.clip), rs.clip)
+                                  : X[static_cast<size_t>(gm) * ldx + k];
+            y = fmaf(x, W[static_cast<size_t>(gn) * K + k], y);
+          }
         }
+        y += bias;
+        if (kElu) y = y > 0.0f ? y : expm1f(y);
+        Y[static_cast<size_t>(gm) * ldy + gn] = y;
       }
+    }
   }
 }
 
@@ -456,17 +533,32 @@ int launch_linear(const float* X, int ldx, const RingSrc& rs, int M, int K, cons
     return mfail(SPI_ERR_INVALID_ARG, "ring-gathered layer needs K % 4 == 0 and 16-byte aligned weights");
   // rows of the ring read as float4: needs ld % 4 == 0 (then rows up to round4(M) <= ld exist)
   const bool ring4 = rs.ring && rs.ld % 4 == 0 && aligned16(rs.ring);
-  if (M >= kBigM && N >= 256 && wvec && xvec) {
-    const dim3 grid((M + kDbRows - 1) / kDbRows, (N + kDbCols - 1) / kDbCols);
-#define SPI_DB(E, S) linear_db_kernel<E, S><<<grid, 256, 0, stream>>>(X, ldx, rs, M, K, W, b, N, Y, ldy)
-    if (ring4) {
-      if (elu) SPI_DB(true, 1); else SPI_DB(false, 1);
+  if (N >= kSpTile && K >= 2 * kSpK && wvec && xvec) {
+    const long long rows = (M + kSpTile - 1) / kSpTile, tiles = rows * ((N + kSpTile - 1) / kSpTile);
+    // A tile per CU or less: two groups share its chunks (900 -> 512 at 2048 rows, 256 tiles: 23.5
+    // us, 26.3 with one; at 4096 rows 46.7, 37.0 with one).  From two 64 x 128 tiles per CU on:
+    // those (16384 rows 122 us, 136 with 64 x 64; 4096 rows, one per CU, 39.7 against 37.0).
+    const int shape = tiles <= kSpGroupTiles ? 0 : tiles < kSpWideTiles ? 1 : 2;
+#define SPI_SP_G(E, S, NN, G) \
+  linear_split_kernel<E, S, NN, G><<<static_cast<int>(rows * ((N + kSpTile * NN - 1) / (kSpTile * NN))), 256 * G, 0, stream>>>( \
+      X, ldx, rs, M, K, W, b, N, Y, ldy)
+#define SPI_SP(E, S)                            \
+  do {                                          \
+    if (shape == 0) SPI_SP_G(E, S, 1, 2);       \
+    else if (shape == 1) SPI_SP_G(E, S, 1, 1);  \
+    else SPI_SP_G(E, S, 2, 1);                  \
+  } while (0)
+    // float2 along the ring's rows: rows up to M rounded to 2 exist (ld even and >= M)
+    const bool ring2 = rs.ring && rs.ld % 2 == 0 && reinterpret_cast<uintptr_t>(rs.ring) % 8 == 0;
+    if (ring2) {
+      if (elu) SPI_SP(true, 1); else SPI_SP(false, 1);
     } else if (rs.ring) {
-      if (elu) SPI_DB(true, 2); else SPI_DB(false, 2);
+      if (elu) SPI_SP(true, 2); else SPI_SP(false, 2);
     } else {
-      if (elu) SPI_DB(true, 0); else SPI_DB(false, 0);
+      if (elu) SPI_SP(true, 0); else SPI_SP(false, 0);
     }
-#undef SPI_DB
+#undef SPI_SP_G
+#undef SPI_SP
   } else {
     const dim3 grid((M + 31) / 32, (N + kCols - 1) / kCols);
     const int split = split_for(M, K, N);

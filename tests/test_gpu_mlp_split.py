@@ -1,0 +1,54 @@
+"""The actor's layers on split products at the edges of their tiles: row counts around a tile, widths
+that leave part of one, inputs of three magnitudes, and non-finite inputs, against float64 and
+against plain float32 products."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _net(dims, seed):
+    from spi_amd.agents.policy import PolicyMLP
+    return PolicyMLP.random(dims[0], dims[-1], dims[1:-1], seed=seed)
+
+
+def _f64(net, x):
+    h = x.astype(np.float64)
+    L = net.layers()
+    for i, (W, b) in enumerate(L):
+        h = h @ W.cpu().numpy().astype(np.float64).T + b.cpu().numpy().astype(np.float64)
+        if i < len(L) - 1:
+            h = np.where(h > 0, h, np.expm1(np.minimum(h, 0)))
+    return h
+
+
+@pytest.mark.parametrize("rows", [1, 63, 64, 65, 200])
+@pytest.mark.parametrize("dims", [(64, 64, 64), (900, 512, 12), (68, 65, 100), (100, 192, 64)])
+@pytest.mark.parametrize("scale", [1e-3, 1.0, 1e4])
+def test_split_layers_match_float64(gpu, rows, dims, scale):
+    import torch
+    net = _net(dims, rows)
+    x = (scale * np.random.default_rng(rows).normal(size=(rows, dims[0]))).astype(np.float32)
+    got = net(torch.from_numpy(x).to(gpu)).cpu().numpy()
+    want = _f64(net, x)
+    # two layers of at most 900 float32 accumulations of random sign: 1e-7 sqrt(900) of the scale
+    assert np.abs(got - want).max() <= 5e-6 * np.abs(want).max()
+
+
+def test_non_finite_inputs_stay_in_their_row(gpu):
+    import torch
+    net = _net((900, 512, 12), 3)
+    x = np.random.default_rng(0).normal(size=(130, 900)).astype(np.float32)
+    clean = net(torch.from_numpy(x).to(gpu)).cpu().numpy()
+    bad = x.copy()
+    bad[5, 7], bad[70, 899], bad[129, 0] = np.inf, np.nan, 3.4e38
+    got = net(torch.from_numpy(bad).to(gpu)).cpu().numpy()
+    keep = [i for i in range(130) if i not in (5, 70, 129)]
+    assert np.array_equal(got[keep], clean[keep])
+    assert np.isnan(got[70]).all() and not np.isfinite(got[5]).any()
+    # one hidden layer of an infinite input: each unit is its weight's sign times infinity
+    one = _net((64, 64), 1)
+    y = np.zeros((1, 64), np.float32)
+    y[0, 3] = np.inf
+    W = one.layers()[0][0].cpu().numpy()
+    assert np.array_equal(one(torch.from_numpy(y).to(gpu)).cpu().numpy()[0], np.sign(W[:, 3]) * np.inf)
