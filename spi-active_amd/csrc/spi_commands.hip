@@ -102,25 +102,27 @@ __device__ __forceinline__ int sampled_slot(const SpiCommandSpec& c, int k) {
 // step's basis once for all of them, each trial's sampled commands go through LDS, and its run of
 // 256 n_dims output words is written in float4 (VEC: n_dims and the steps of a trial make every
 // run a multiple of 16 bytes).  Bound by the output: 1024 trials x 1250 steps x 14 (71.7 MB) in
-// 28 us; 45 us with a basis per (trial, step) and all 14 commands through LDS.
+// 26 us; 45 us with a basis per (trial, step) and all 14 commands through LDS.
+typedef float FloatX4 __attribute__((ext_vector_type(4)));
 constexpr int kStepThreads = 256, kTrialsPerBlock = 8;
 template <bool VEC>
 __global__ __launch_bounds__(kStepThreads) void command_trials_kernel(SpiCommandSpec c, const float* __restrict__ params,
                                                                       int n_trials, int n_params, int T, int per,
                                                                       float* __restrict__ out) {
   __shared__ float val[SPI_MAX_COMMAND_DIMS * (kStepThreads + 1)];   // sampled slots, then the defaults
-  __shared__ int at[SPI_MAX_COMMAND_DIMS], inc[SPI_MAX_COMMAND_DIMS];
+  __shared__ int2 at[SPI_MAX_COMMAND_DIMS];            // dimension k of step s is val[at[k].x + at[k].y s]
   const int tid = threadIdx.x, step = blockIdx.x * kStepThreads + tid, nd = c.n_dims;
   const int n_steps = min(kStepThreads, T - static_cast<int>(blockIdx.x) * kStepThreads);
   float* def = val + SPI_MAX_COMMAND_DIMS * kStepThreads;
   if (tid < nd) {
     const int d = sampled_slot(c, tid);
-    at[tid] = d >= 0 ? d * kStepThreads : SPI_MAX_COMMAND_DIMS * kStepThreads + tid;
-    inc[tid] = d >= 0;
+    at[tid] = d >= 0 ? make_int2(d * kStepThreads, 1) : make_int2(SPI_MAX_COMMAND_DIMS * kStepThreads + tid, 0);
     def[tid] = c.default_cmd[tid];
   }
   const StepBasis sb = step_basis(c, min(step, T - 1));
   const int b0 = blockIdx.y * per, b1 = min(b0 + per, n_trials);
+  // step and dimension of this thread's first float4, and what 256 float4 further adds
+  const int sv = 4 * tid / nd, kv = 4 * tid - sv * nd, ds = 4 * kStepThreads / nd, dk = 4 * kStepThreads - ds * nd;
   for (int b = b0; b < b1; ++b) {
     const float* p = params + static_cast<size_t>(b) * n_params;
     for (int d = 0; d < c.n_sampled; ++d) val[d * kStepThreads + tid] = sampled_command(c, sb, p, d, c.sampled_idx[d]);
@@ -128,21 +130,26 @@ __global__ __launch_bounds__(kStepThreads) void command_trials_kernel(SpiCommand
     float* o = out + (static_cast<size_t>(b) * T + static_cast<size_t>(blockIdx.x) * kStepThreads) * nd;
     const int n_out = n_steps * nd;
     if (VEC) {
-      float4* o4 = reinterpret_cast<float4*>(o);
+      FloatX4* o4 = reinterpret_cast<FloatX4*>(o);
+      int s0 = sv, k0 = kv;
       for (int e = tid; 4 * e < n_out; e += kStepThreads) {
         float v[4];
-        int s = 4 * e / nd, k = 4 * e - s * nd;
+        int s = s0, k = k0;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          v[q] = val[at[k] + inc[k] * s];
+          const int2 a = at[k];
+          v[q] = val[a.x + a.y * s];
           if (++k == nd) { k = 0; ++s; }
         }
-        o4[e] = make_float4(v[0], v[1], v[2], v[3]);
+        __builtin_nontemporal_store(FloatX4{v[0], v[1], v[2], v[3]}, o4 + e);   // written once, not read here
+        s0 += ds;
+        k0 += dk;
+        if (k0 >= nd) { k0 -= nd; ++s0; }
       }
     } else {
       for (int e = tid; e < n_out; e += kStepThreads) {
         const int s = e / nd, k = e - s * nd;
-        o[e] = val[at[k] + inc[k] * s];
+        o[e] = val[at[k].x + at[k].y * s];
       }
     }
     __syncthreads();

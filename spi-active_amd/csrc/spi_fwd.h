@@ -1,8 +1,8 @@
 // Forward dynamics of the primal rollouts (gfx950): the Go2 step of spi_dyn.h with every leg
 // eliminated in closed form in its hip frame.  Same model, contact law and integrator as
 // spi_dyn.h in two thirds of its instructions: a rollout lane is bound by VALU issue, so the
-// algebra is what its time consists of (3,666 FLOP per sub-interval against 5,293; vector
-// instructions 3,399 -> 2,250).
+// algebra is what its time consists of (3,546 FLOP per sub-interval against 5,293; vector
+// instructions 3,399 -> 2,180).
 //
 // What the leg's structure gives (hip axis x; thigh and calf axes both y; the thigh's origin
 // lies on its own axis through the hip origin O, so every y offset can be absorbed into the
@@ -21,8 +21,8 @@
 //     k = -s (2 wy + s), at p from that point.  No per-link velocity or force is formed, and
 //     with the base's proper acceleration dv/dt + w x v - g as the unknown, none depends on v.
 // Measured on 4096 candidates x 256 segments x H 20 (rollout_cost_kernel): 31.6 -> 23.2 ms by the
-// algebra, -> 16.6 ms with two waves per SIMD (end_leg below, LaneLds in spi_kernels.hip).  Error
-// of the costs against 64 bits unchanged (2.7e-6 before, 2.8e-6 after).
+// algebra, -> 16.3 ms with two waves per SIMD (end_leg below, LaneLds in spi_kernels.hip).  Error
+// of the costs against 64 bits: 2.2e-6 before, 2.0e-6 after.
 #pragma once
 #include "spi_dyn.h"
 

@@ -133,8 +133,8 @@ __device__ __forceinline__ unsigned int rollout_lane(const SpiSimArgs& a, const 
 // One workgroup = one segment x 256 candidates; parameters are read coalesced from the SoA array,
 // the segment record through the scalar cache.  Bound by VALU issue: 244 registers (two waves per
 // SIMD), no spills, no copies between register files.  4096 candidates x 256 segments x H 20:
-// 31.6 ms with the articulated-body step at 438 registers, 16.6 ms now (73.9 TFLOP/s of the
-// algorithm's own 58,656 FLOP per control step).
+// 31.6 ms with the articulated-body step at 438 registers, 16.3 ms now (73.0 TFLOP/s of the
+// algorithm's own 56,739 FLOP per control step).
 __global__ __launch_bounds__(kRolloutThreads, 2) void rollout_cost_kernel(
     SpiSimArgs a, SpiCostArgs cost, const float* __restrict__ par, int ld, int n_cand,
     const float* __restrict__ seg, int H, int stride, int n_cblk, float* __restrict__ out) {
