@@ -35,8 +35,8 @@ METRIC = "env-steps/s, sysID solves/s at ≤1% param error; p50/p99 solve latenc
 FLOPS_PER_CONTROL_STEP = 56739.0
 PEAK_FP32_TFLOPS = 157.3          # MI355X published FP32 (vector) peak
 # HBM bytes per rollout_cost_kernel launch of this workload: rocprofv3 --pmc FETCH_SIZE
-# (2,359.5 KiB, x 2.000 from a 256 MiB copy's reading) + WRITE_SIZE (4,096.0 KiB, x 1.000).
-TRAFFIC_BYTES_PER_LAUNCH = 9026560
+# (2,797.1 KiB, x 2.000 from a 256 MiB copy's reading) + WRITE_SIZE (4,096.0 KiB, x 1.000).
+TRAFFIC_BYTES_PER_LAUNCH = 9922688
 
 N_SAMPLES, N_SEG, HORIZON, ITERS = 4096, 256, 20, 12
 FIXTURE = os.path.join(ROOT, "tests", "golden", "c1_fp64_minimiser.npz")
@@ -375,7 +375,7 @@ def _rows_from_prior(prior, n, seed=0):
 
 
 def cpu_baseline(sim, seg_packed, prior, weights, target_s=10.0):
-    """The GPU kernel's algorithm on the host: spi_dyn.h built for x86-64-v3 with OpenMP
+    """The GPU kernel's algorithm on the host: spi_fwd.h built for x86-64-v3 with OpenMP
     (tests/host_dyn/spi_rollout_cpu.cpp), over all the cores this process may use, on a bounded
     sample of the workload's candidates (all 256 segments x H 20, about target_s seconds)."""
     import ctypes
@@ -407,7 +407,7 @@ def cpu_baseline(sim, seg_packed, prior, weights, target_s=10.0):
         dt, used = run(n)
         steps = n * n_seg * HORIZON
         return {"value": round(steps / dt, 1), "unit": "env-steps/s", "cores": used, "kind": "port",
-                "algorithm": "same as the GPU kernel: spi_dyn.h built for the host (x86-64-v3, OpenMP), one "
+                "algorithm": "same as the GPU kernel: spi_fwd.h built for the host (x86-64-v3, OpenMP), one "
                              "rollout per thread iteration",
                 "cores_visible": visible,
                 "sample": f"{n} of {N_SAMPLES} CEM candidates x {n_seg} segments x H={HORIZON} "

@@ -53,7 +53,7 @@ def _host_cores() -> int:
 
 
 def _cpu_rollout_lib():
-    """The rollout kernels' algorithm built for the host (spi_dyn.h, x86-64-v3, OpenMP:
+    """The rollout kernels' algorithm built for the host (spi_fwd.h, x86-64-v3, OpenMP:
     tests/host_dyn/spi_rollout_cpu.cpp), the same-algorithm CPU baseline."""
     import ctypes
     import os

@@ -1,21 +1,22 @@
-// Host-CPU baseline with the GPU kernel's own algorithm: spi_dyn.h (PD law + motor model,
-// articulated-body dynamics specialised to the Go2 tree, penalty contact, semi-implicit Euler
-// with torque held over the sub-intervals) built for x86 and run over OpenMP threads, one
+// Host-CPU baseline with the GPU kernel's own algorithm: spi_fwd.h over spi_dyn.h (PD law + motor
+// model, forward dynamics by leg elimination, penalty contact, semi-implicit Euler with torque
+// held over the sub-intervals) built for x86 and run over OpenMP threads, one
 // (candidate, segment) rollout per loop iteration, scored like rollout_cost_kernel.  bench.py
 // times it beside the GPU; nothing in the library runs it.
 #include <cstring>
 
 #include <omp.h>
 
-#include "spi_dyn.h"
+#include "spi_fwd.h"
 
 using namespace spi;
 
 namespace {
 LaneParams lane_params(const float* par, int ld, int i) {
   LaneParams lp;
-  lp.base = make_base_inertia(par[0 * ld + i], par[1 * ld + i], par[2 * ld + i], par[3 * ld + i], par[4 * ld + i],
-                              par[5 * ld + i], par[6 * ld + i], par[7 * ld + i], par[8 * ld + i], par[9 * ld + i]);
+  lp.base = base_with_legs(make_base_inertia(par[0 * ld + i], par[1 * ld + i], par[2 * ld + i], par[3 * ld + i],
+                                             par[4 * ld + i], par[5 * ld + i], par[6 * ld + i], par[7 * ld + i],
+                                             par[8 * ld + i], par[9 * ld + i]));
   for (int l = 0; l < 4; ++l) {
     lp.kp_s[l] = par[(10 + l) * ld + i];
     lp.kd_s[l] = par[(14 + l) * ld + i];
@@ -76,7 +77,7 @@ extern "C" int spi_cpu_rollout_cost(const SpiSimArgs* a, const SpiCostArgs* cost
         for (int d = 0; d < as.decimation; ++d) {
           float tau[12];
           control_torques(as, lp, rec, st, tau);
-          physics_step(as, lp, st, tau, nullptr);
+          physics_step_elim(as, LaneRegs{lp, tau}, st, nullptr);
         }
         if (cost->mode == SPI_COST_TRACKING || t == H - 1) acc += step_cost(*cost, st, rec + 12);
         const float nrm = state_norm(st);
