@@ -151,7 +151,7 @@ __global__ __launch_bounds__(kRolloutThreads, 2) void rollout_cost_kernel(
   *o = rollout_lane<1>(a, cost, ln, seg + static_cast<size_t>(s) * stride, H);
 }
 
-// rollout_cost_kernel with four lanes per candidate, one per leg (spi_dyn_leg.h): one
+// rollout_cost_kernel with four lanes per candidate, one per leg (spi_fwd_leg.h): one
 // workgroup = one segment x 64 candidates.  For batches that leave most SIMDs idle (a mass
 // landscape, a small job), the rollout's latency drops at the price of more instructions in
 // total; same costs up to the order of the legs' sums.

@@ -113,7 +113,7 @@ __global__ __launch_bounds__(kPolThreads) void policy_step_kernel(SpiSimArgs a, 
   state_to_root(st, dst, dst + 13, dst + 25, 1);
 }
 
-// policy_step_kernel with four lanes per env (lane % 4 = leg, spi_dyn_leg.h): the same step,
+// policy_step_kernel with four lanes per env (lane % 4 = leg, spi_fwd_leg.h): the same step,
 // for batches too small to fill the SIMDs with one env per lane.
 __device__ __forceinline__ float pick4(int l, float x0, float x1, float x2, float x3) {
   return l == 0 ? x0 : (l == 1 ? x1 : (l == 2 ? x2 : x3));
