@@ -58,17 +58,32 @@ class SegmentStore:
         _lib.require_gpu()
         self.device = torch.device(device)
         self.trajectories: List[Trajectory] = []
-        self._joined = None           # (states [R, 37], actions [R, 12], first row of each trajectory)
-        self._first_dev = None        # the first rows on the device
+        # (states [R, 37], actions [R, 12], first row of each trajectory, the same on the device),
+        # and the stream that they were built on
+        self._joined = None
 
     def _joined_buffers(self):
-        """All trajectories back to back in one device buffer (rebuilt after an add)."""
-        if self._joined is None or len(self._joined[2]) != len(self.trajectories):
-            starts = np.cumsum([0] + [tr.n_steps for tr in self.trajectories])[:-1]
-            self._first_dev = torch.from_numpy(np.minimum(starts, 2 ** 31 - 1).astype(np.int32)).to(self.device)
-            self._joined = (torch.cat([tr.states for tr in self.trajectories]),
-                            torch.cat([tr.actions for tr in self.trajectories]), starts)
-        return self._joined
+        return self._joined_with_rows()[:3]
+
+    def _joined_with_rows(self):
+        """All trajectories back to back in one device buffer (rebuilt after an add).  A later call
+        may run on any stream and cannot order itself after a build that it does not know of, so
+        the build is complete before its buffers are kept; a call on another stream than the
+        build's marks them as used there, so that a rebuild does not hand their memory on early."""
+        stream = torch.cuda.current_stream(self.device)
+        joined = self._joined
+        if joined is None or len(joined[0][2]) != len(self.trajectories):
+            trs = list(self.trajectories)
+            starts = np.cumsum([0] + [tr.n_steps for tr in trs])[:-1]
+            kept = (torch.cat([tr.states for tr in trs]), torch.cat([tr.actions for tr in trs]), starts,
+                    torch.from_numpy(np.minimum(starts, 2 ** 31 - 1).astype(np.int32)).to(self.device))
+            stream.synchronize()
+            self._joined = joined = (kept, stream)
+        kept, built_on = joined
+        if stream != built_on:
+            for t in (kept[0], kept[1], kept[3]):
+                t.record_stream(stream)
+        return kept
 
     def add_arrays(self, states: np.ndarray, actions: np.ndarray, kp: float = 20.0, kd: float = 0.5,
                    name: Optional[str] = None) -> int:
@@ -97,7 +112,7 @@ class SegmentStore:
         if n == 0:
             raise ValueError("no trajectory is longer than the horizon")
         out = torch.empty((n, segment_stride(horizon)), dtype=torch.float32, device=self.device)
-        states, actions, first = self._joined_buffers()
+        states, actions, first, first_dev = self._joined_with_rows()
         if states.shape[0] >= 2 ** 31:
             raise ValueError("the store holds more than 2^31 - 1 trajectory rows")
         # every window of every trajectory: the kernel finds the rows itself; a choice of
@@ -113,7 +128,7 @@ class SegmentStore:
         L = _lib.lib()
         if whole:
             rc = L.spi_pack_windows_store(_lib.ptr(states), _lib.ptr(actions), states.shape[0],
-                                          _lib.ptr(self._first_dev, torch.int32), len(which), n, horizon, _lib.ptr(out),
+                                          _lib.ptr(first_dev, torch.int32), len(which), n, horizon, _lib.ptr(out),
                                           _lib.stream())
             _lib.check(rc, "spi_pack_windows_store")
         L.spi_window_index(len(which), *[a.ctypes.data for a in table], ends.ctypes.data, src.ctypes.data,
