@@ -7,7 +7,7 @@
 // tile, rows of X and the weight rows staged through LDS in K chunks of 64 (even columns, then odd
 // ones, 65 words per row, so the operand reads of a wavefront hit 64 distinct banks).  Strict IEEE
 // float32 (no fast-math).
-// The actor (900 -> 512 -> 256 -> 128 -> 12): 2048 rows 63 -> 50 us, 16384 rows 222 -> 175 us.
+// The actor (900 -> 512 -> 256 -> 128 -> 12): 2048 rows 63 -> 54 us, 16384 rows 222 -> 205 us.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -285,29 +285,40 @@ int split_for(int M, int K, int N) {
   return tiles <= 128 ? 4 : 2;
 }
 
-// float32 products on the bf16 matrix pipe.  A float is exactly the sum of three bf16 values (its
-// 24 significant bits in 8 + 8 + 8, each part truncated), so a product is nine bf16 products;
-// the six largest are kept (the dropped ones are below 2^-22 of it) and accumulated in float32:
-// six v_mfma_f32_32x32x16_bf16 of 32 cycles replace eight v_mfma_f32_32x32x2_f32 of 64.  The
-// leading products and the five small ones have an accumulator each, so the leading one adds 57
-// times where the float32 pipe added 450 times for 900 inputs: the error of the whole actor against 64
-// bits fell from 3.3e-7 .. 6.4e-7 to 2.5e-7 .. 3.5e-7 (batches of 16 .. 16384 rows).
+// float32 products on the bf16 matrix pipe.  A float is exactly the sum of three bf16 values (each
+// part rounded to nearest, the next one takes what it left), so a product is nine bf16 products.
+// Eight are formed; the ninth, of the two last parts, is below 2^-34 of the product and no larger in
+// sum than the rounding of the accumulators.  (With the six largest of truncated parts an output of
+// one non-zero input was off by up to 4.1e-7 of itself, always towards zero; now as by one float32
+// rounding, 6.0e-8.)  Operands are scaled by 2^16, so that the last part of any float is a bf16,
+// subnormal floats' too: unscaled, inputs or weights of 1e-36 lost 5e-5 of the result.  Eight
+// v_mfma_f32_32x32x16_bf16 of 32 cycles replace eight v_mfma_f32_32x32x2_f32 of 64.
+// The leading products and the seven small ones have an accumulator each, so the leading one adds
+// 57 times where the float32 pipe added 450 times for 900 inputs: relative error of such a layer
+// against 64 bits 3.8e-7 on the float32 pipe, 1.2e-7 here; with 1, 4 and 16 non-zero inputs 2.53e-8,
+// 4.2e-8 and 6.1e-8 there, 2.53e-8, 3.6e-8 and 4.0e-8 here.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+constexpr float kOperandScale = 65536.0f, kResultScale = 1.0f / (kOperandScale * kOperandScale);
 struct Split4 { uint2 p[3]; };      // the three parts of four consecutive inputs
+__device__ __forceinline__ unsigned bf16_pair(float a, float b) {   // v_cvt_pk_bf16_f32, a in the low half
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(floatx2{a, b}, bf16x2));
+}
 __device__ __forceinline__ Split4 split4(const float* x) {
-  unsigned u[3][4];
+  float r[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    u[0][i] = __float_as_uint(x[i]);
-    const float r = x[i] - __uint_as_float(u[0][i] & 0xffff0000u);
-    u[1][i] = __float_as_uint(r);
-    u[2][i] = __float_as_uint(r - __uint_as_float(u[1][i] & 0xffff0000u));
-  }
+  for (int i = 0; i < 4; ++i) r[i] = kOperandScale * x[i];
   Split4 s;
 #pragma unroll
-  for (int q = 0; q < 3; ++q)   // the high halves of two words
-    s.p[q] = make_uint2(__builtin_amdgcn_perm(u[q][1], u[q][0], 0x07060302u),
-                        __builtin_amdgcn_perm(u[q][3], u[q][2], 0x07060302u));
+  for (int q = 0; q < 3; ++q) {
+    s.p[q] = make_uint2(bf16_pair(r[0], r[1]), bf16_pair(r[2], r[3]));
+    if (q == 2) break;
+    r[0] -= __uint_as_float(s.p[q].x << 16);
+    r[1] -= __uint_as_float(s.p[q].x & 0xffff0000u);
+    r[2] -= __uint_as_float(s.p[q].y << 16);
+    r[3] -= __uint_as_float(s.p[q].y & 0xffff0000u);
+  }
   return s;
 }
 
@@ -331,7 +342,7 @@ __device__ __forceinline__ void tile_of(int id, int n_tiles, int n_col, int* row
 // LDS rows are four 16-byte units of 8 columns, unit u of row r at u ^ (r / 2) % 4: the 16-byte
 // operand reads of 8 rows and the 8-byte stores of a row's columns each cover the banks once.
 // Lane l supplies row l % 32 and columns 8 (l / 32) .. + 7 of both operands.
-// A wavefront issues 12 kN MFMAs (32 cycles each) and splits 8 (1 + kN) values (5.5 vector
+// A wavefront issues 16 kN MFMAs (32 cycles each) and splits 8 (1 + kN) values (6.5 vector
 // instructions of 4 cycles each) per chunk, and the two do not overlap on a SIMD: kN = 2 halves
 // the splitting per product where the tiles still fill the chip.  kG groups of 4 wavefronts take
 // alternate chunks and add up in group order at the end: for batches of one tile per CU, whose
@@ -339,8 +350,8 @@ __device__ __forceinline__ void tile_of(int id, int n_tiles, int n_col, int* row
 // kSrc 0: X row-major; 1: X gathered from a RingSrc in blocks of 2 rows x 4 columns, float2 along
 // the rows (lines 8-byte aligned, ld even); 2: the same blocks in scalar loads.  The accumulation
 // order does not depend on the source: dense and ring input give the same bits.
-// A result that is not finite (an infinite or NaN input has no finite parts) is formed again from
-// float32 products.
+// A result that is not finite (an infinite or NaN operand, or one of 2^112 and more, has no finite
+// parts) is formed again from float32 products.
 constexpr int kSpTile = 64, kSpK = 32;
 constexpr int kSpGroupTiles = 256, kSpWideTiles = 1024;   // tiles of 64 x 64
 template <bool kElu, int kSrc, int kN, int kG>
@@ -452,8 +463,10 @@ __global__ __launch_bounds__(256 * kG, 2) void linear_split_kernel(const float* 
 #define SPI_MM(A, P, Q)                                                                                  \
   _Pragma("unroll") for (int n = 0; n < kN; ++n)                                                         \
       A[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[P], w[n][Q], A[n], 0, 0, 0);
-      SPI_MM(lo, 2, 0)
+      SPI_MM(lo, 2, 1)
       SPI_MM(hi, 0, 0)
+      SPI_MM(lo, 1, 2)
+      SPI_MM(lo, 2, 0)
       SPI_MM(lo, 0, 2)
       SPI_MM(lo, 1, 1)
       SPI_MM(lo, 1, 0)
@@ -501,6 +514,7 @@ __global__ __launch_bounds__(256 * kG, 2) void linear_split_kernel(const float* 
       if (gm < M) {
         float y = hi[n][r] + lo[n][r];
         for (int g = 1; g < kG; ++g) y += reinterpret_cast<const float*>(lds)[(((g - 1) * kN + n) * 16 + r) * 256 + tid];
+        y *= kResultScale;
         if (!isfinite(y)) {
           y = 0.0f;
           for (int k = 0; k < K; ++k) {

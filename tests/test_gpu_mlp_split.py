@@ -52,3 +52,44 @@ def test_non_finite_inputs_stay_in_their_row(gpu):
     y[0, 3] = np.inf
     W = one.layers()[0][0].cpu().numpy()
     assert np.array_equal(one(torch.from_numpy(y).to(gpu)).cpu().numpy()[0], np.sign(W[:, 3]) * np.inf)
+
+
+def _one_layer(W):
+    from spi_amd.agents.policy import PolicyMLP
+    return PolicyMLP([(W, np.zeros(W.shape[0], np.float32))])
+
+
+@pytest.mark.parametrize("non_zero", [1, 4])
+def test_rows_of_few_inputs_round_like_float32(gpu, non_zero):
+    """A sum of n float32 products is off by at most n roundings of 2^-24 of the products' magnitudes,
+    and a single product by one."""
+    import torch
+    rng = np.random.default_rng(non_zero)
+    W = rng.normal(size=(512, 900)).astype(np.float32)
+    x = np.zeros((520, 900), np.float32)
+    for row in x:
+        row[rng.choice(900, non_zero, replace=False)] = rng.normal(size=non_zero)
+    got = _one_layer(W)(torch.from_numpy(x).to(gpu)).cpu().numpy().astype(np.float64)
+    x, W = x.astype(np.float64), W.astype(np.float64)
+    assert (np.abs(got - x @ W.T) <= 1.02 * non_zero * 2.0 ** -24 * (np.abs(x) @ np.abs(W).T)).all()
+
+
+def test_positive_sums_are_not_biased(gpu):
+    """130 x 512 sums of 900 positive products: their mean relative error is far below a rounding."""
+    import torch
+    rng = np.random.default_rng(5)
+    x, W = (np.abs(rng.normal(size=(n, 900))).astype(np.float32) for n in (130, 512))
+    got = _one_layer(W)(torch.from_numpy(x).to(gpu)).cpu().numpy().astype(np.float64)
+    assert abs((got / (x.astype(np.float64) @ W.astype(np.float64).T) - 1).mean()) < 2.0 ** -27
+
+
+@pytest.mark.parametrize("scale_x,scale_w", [(1e-36, 1), (1, 1e-36), (1e-36, 1e30), (1e30, 1e-36), (1e-39, 1e30),
+                                             (1e37, 1e-37), (1e18, 1e18), (1e25, 1e5)])
+def test_magnitudes_over_the_whole_range(gpu, scale_x, scale_w):
+    """64 products of operands near either end of float32: 64 roundings of 2^-24 would be 4e-6."""
+    import torch
+    rng = np.random.default_rng(9)
+    x, W = (scale_x * rng.normal(size=(70, 64))).astype(np.float32), (scale_w * rng.normal(size=(64, 64))).astype(np.float32)
+    got = _one_layer(W)(torch.from_numpy(x).to(gpu)).cpu().numpy().astype(np.float64)
+    want = x.astype(np.float64) @ W.astype(np.float64).T
+    assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
