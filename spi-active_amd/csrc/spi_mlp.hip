@@ -351,7 +351,9 @@ __device__ __forceinline__ void tile_of(int id, int n_tiles, int n_col, int* row
 // the rows (lines 8-byte aligned, ld even); 2: the same blocks in scalar loads.  The accumulation
 // order does not depend on the source: dense and ring input give the same bits.
 // A result that is not finite (an infinite or NaN operand, or one of 2^112 and more, has no finite
-// parts) is formed again from float32 products.
+// parts) is formed again on the float32 pipe, by its wavefront together: 16 bad rows of 2048 1220 us
+// with a loop per element, 88 us so
+// (66 where every batch took the float32 pipe).
 constexpr int kSpTile = 64, kSpK = 32;
 constexpr int kSpGroupTiles = 256, kSpWideTiles = 1024;   // tiles of 64 x 64
 template <bool kElu, int kSrc, int kN, int kG>
@@ -503,29 +505,67 @@ __global__ __launch_bounds__(256 * kG, 2) void linear_split_kernel(const float* 
     __syncthreads();
     if (grp > 0) return;
   }
+  // results of the wavefront's tile n that are not finite over again from float32 products, K in
+  // steps of 8 (4 columns per half), four steps multiplied while four are in flight; a row's results
+  // never depend on the rows beside it
+  auto in_float32 = [&](int n, float* y) {
+    const int gm = min(m0 + wr + col, M - 1), gn = min(n0 + wc + 32 * n + col, N - 1);
+    floatx16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+    struct Step { float x[4][4], w[4][4]; };
+    auto load = [&](Step& s, int k0) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int k = k0 + 8 * j + 4 * half;
+        const bool in = k < K;
+        load4(s.w[j], W + static_cast<size_t>(gn) * K + k, in);
+        if (!kRing) {
+          load4(s.x[j], X + static_cast<size_t>(gm) * ldx + k, in);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) s.x[j][e] = in ? rs.ring[static_cast<size_t>(Kr[k + e]) * rs.ld + gm] : 0.0f;
+        }
+      }
+    };
+    Step s;
+    load(s, 0);
+    for (int k0 = 0; k0 < K; k0 += 32) {
+      Step t;
+      load(t, k0 + 32);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          acc = __builtin_amdgcn_mfma_f32_32x32x2f32(kRing ? fminf(fmaxf(s.x[j][e], -rs.clip), rs.clip) : s.x[j][e],
+                                                     s.w[j][e], acc, 0, 0, 0);
+      s = t;
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) y[r] = isfinite(y[r]) ? y[r] : acc[r];
+  };
 #pragma unroll
   for (int n = 0; n < kN; ++n) {
-    const int gn = n0 + wc + 32 * n + col;
-    if (gn >= N) continue;
-    const float bias = b[gn];
+    const int gn = n0 + wc + 32 * n + col, gm0 = m0 + wr + 4 * half;   // row of register r: gm0 + 8 (r / 4) + r % 4
+    float y[16];
+    bool finite = true;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const int gm = m0 + wr + 8 * (r >> 2) + 4 * half + (r & 3);
-      if (gm < M) {
-        float y = hi[n][r] + lo[n][r];
-        for (int g = 1; g < kG; ++g) y += reinterpret_cast<const float*>(lds)[(((g - 1) * kN + n) * 16 + r) * 256 + tid];
-        y *= kResultScale;
-        if (!isfinite(y)) {
-          y = 0.0f;
-          for (int k = 0; k < K; ++k) {
-            const float x = kRing ? fminf(fmaxf(rs.ring[static_cast<size_t>(Kr[k]) * rs.ld + gm], -rs.clip), rs.clip)
-                                  : X[static_cast<size_t>(gm) * ldx + k];
-            y = fmaf(x, W[static_cast<size_t>(gn) * K + k], y);
-          }
+      y[r] = hi[n][r] + lo[n][r];
+      for (int g = 1; g < kG; ++g) y[r] += reinterpret_cast<const float*>(lds)[(((g - 1) * kN + n) * 16 + r) * 256 + tid];
+      y[r] *= kResultScale;
+      finite = finite && isfinite(y[r]);
+    }
+    if (__any(!finite)) in_float32(n, y);
+    if (gn < N) {
+      const float bias = b[gn];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int gm = gm0 + 8 * (r >> 2) + (r & 3);
+        if (gm < M) {
+          const float v = y[r] + bias;
+          Y[static_cast<size_t>(gm) * ldy + gn] = kElu ? (v > 0.0f ? v : expm1f(v)) : v;
         }
-        y += bias;
-        if (kElu) y = y > 0.0f ? y : expm1f(y);
-        Y[static_cast<size_t>(gm) * ldy + gn] = y;
       }
     }
   }

@@ -93,3 +93,66 @@ def test_magnitudes_over_the_whole_range(gpu, scale_x, scale_w):
     got = _one_layer(W)(torch.from_numpy(x).to(gpu)).cpu().numpy().astype(np.float64)
     want = x.astype(np.float64) @ W.astype(np.float64).T
     assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
+
+
+def _times(f, n=7):
+    import torch
+    out = []
+    for _ in range(n + 2):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        f()
+        b.record()
+        b.synchronize()
+        out.append(a.elapsed_time(b))
+    return min(out[2:])
+
+
+def test_non_finite_rows_do_not_stall_the_batch(gpu):
+    """Sixteen NaN rows among 2048: no more than a few times the clean batch."""
+    import torch
+    net = _net((900, 512, 256, 128, 12), 4)
+    x = torch.randn((2048, 900), device=gpu)
+    bad = x.clone()
+    bad[:48:3, 5] = float("nan")
+    assert _times(lambda: net(bad)) < 4 * _times(lambda: net(x))
+
+
+# a tile shape each: two groups, one group, 128 columns (70 and 192: part of a tile)
+@pytest.mark.parametrize("rows,width", [(130, 70), (6000, 192), (22000, 192)])
+@pytest.mark.parametrize("ring", [None, 0, 1])
+def test_non_finite_and_huge_operands_in_every_tile_shape(gpu, rows, width, ring):
+    """inf, NaN and 3e38 in single rows against float64 (an infinite sum stays infinite, a NaN one
+    NaN), dense and from a ring (lines aligned, and one row on); the rows between are as without them."""
+    import torch
+    rng = np.random.default_rng(rows)
+    K = 68
+    net = _one_layer(rng.normal(size=(width, K)).astype(np.float32))
+    W = net.layers()[0][0].cpu().numpy().astype(np.float64)
+    x = rng.normal(size=(rows, K)).astype(np.float32)
+    bad = x.copy()
+    at = {5: np.inf, 63: -np.inf, 64: np.nan, rows // 2: 3e38, rows - 1: np.inf}
+    for i, (r, v) in enumerate(at.items()):
+        bad[r, (7 * i) % K] = v
+
+    def run(a):
+        if ring is None:
+            return net(torch.from_numpy(a).to(gpu)).cpu().numpy()
+        buf = torch.zeros((3, K, rows + 2 + ring), device=gpu)     # the newest line holds the rows
+        buf[1, :, ring:ring + rows] = torch.from_numpy(a.T.copy()).to(gpu)
+        kmap = torch.stack([torch.zeros(K, dtype=torch.int32), torch.arange(K, dtype=torch.int32)], 1).to(gpu).contiguous()
+        return net.forward_ring(buf, 1, kmap, 3.3e38, rows, row0=ring).cpu().numpy()
+
+    clean, got = run(x), run(bad)
+    keep = np.setdiff1d(np.arange(rows), list(at))
+    assert np.array_equal(got[keep], clean[keep])
+    if ring is not None:
+        bad = np.where(np.isnan(bad), np.float32(-3.3e38), np.clip(bad, np.float32(-3.3e38), np.float32(3.3e38)))
+    with np.errstate(all="ignore"):
+        for r in at:
+            want = (bad[r].astype(np.float64)[None] * W).sum(1).astype(np.float32)
+            finite = np.isfinite(want)
+            assert np.array_equal(np.isnan(want), np.isnan(got[r])) and np.array_equal(want[~finite], got[r][~finite], equal_nan=True)
+            assert np.allclose(got[r][finite], want[finite], rtol=1e-5, atol=0)
+    # 68 terms of about 1, 2e-6 of their sum's scale
+    assert np.abs(clean - x.astype(np.float64) @ W.T).max() < 1e-4
