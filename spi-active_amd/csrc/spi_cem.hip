@@ -107,8 +107,7 @@ __global__ void reduce_segments_kernel(const float* __restrict__ cs, const float
 constexpr int kCemThreads = 1024;
 
 constexpr int kSelectMax = 1024;   // elites that the selection handles; more are sorted
-constexpr int kListMax = 2048;     // candidates up to the threshold (its ties included)
-static_assert(kSelectMax <= kListMax && 2 * kListMax <= SPI_MAX_CEM_SAMPLES, "val holds the elites and the ranks");
+static_assert(4 * kSelectMax <= SPI_MAX_CEM_SAMPLES, "val holds the elites, their ranks and their list");
 
 // Order of the ranking as unsigned integers: ascending cost, NaN as +inf, -0 as 0.
 __device__ __forceinline__ unsigned order_bits(float c) {
@@ -119,13 +118,15 @@ __device__ __forceinline__ unsigned order_bits(float c) {
 
 // The n_elite lowest (cost, index) pairs in ascending order into val[0 .. n_elite), for n_elite <=
 // kSelectMax: the n_elite-th lowest cost by four 8-bit counting passes over the keys, then the
-// candidates up to it ranked against each other.  False (val undefined) if more than kListMax
-// candidates tie up to the threshold.  A sort of all 4096 pairs took 78 barriers of about a
-// microsecond each; this takes a dozen.  Called by a whole workgroup.
-__device__ bool select_elites(const float* key, int* val, unsigned long long* list, int n, int n_elite) {
+// n_elite candidates up to it ranked against each other.  Of those that tie with the threshold the
+// lowest indices are taken, counted in index order where there are more than fit.  val also holds the
+// list and the ranks, so that two workgroups' LDS fits a CU.  Called by a whole workgroup.
+__device__ __forceinline__ void select_elites(const float* key, int* val, int n, int n_elite) {
   __shared__ int hist[256];
   __shared__ unsigned prefix_s;
-  __shared__ int want_s, count_s;
+  __shared__ int want_s, ties_s, count_s;
+  int* rank = val + kSelectMax;
+  unsigned long long* list = reinterpret_cast<unsigned long long*>(val + 2 * kSelectMax);
   const int tid = threadIdx.x, lane = tid & 63;
   unsigned prefix = 0;     // digits of the threshold so far
   int want = n_elite;      // its rank among the keys that share them
@@ -169,6 +170,7 @@ __device__ bool select_elites(const float* key, int* val, unsigned long long* li
         while (below + h[k] < want) below += h[k++];
         prefix_s = (prefix << 8) | static_cast<unsigned>(4 * lane + k);
         want_s = want - below;
+        ties_s = h[k];
       }
       if (tid == 0) count_s = 0;
     }
@@ -176,20 +178,33 @@ __device__ bool select_elites(const float* key, int* val, unsigned long long* li
     prefix = prefix_s;
     want = want_s;
   }
+  auto entry = [&](unsigned u, int i) { return (static_cast<unsigned long long>(u) << 32) | static_cast<unsigned>(i); };
+  const bool all_ties = ties_s == want;
   for (int i = tid; i < n; i += kCemThreads) {
     const unsigned u = order_bits(key[i]);
-    if (u <= prefix) {
-      const int at = atomicAdd(&count_s, 1);
-      if (at < kListMax) list[at] = (static_cast<unsigned long long>(u) << 32) | static_cast<unsigned>(i);
+    if (u < prefix || (all_ties && u == prefix)) list[atomicAdd(&count_s, 1)] = entry(u, i);
+  }
+  const int m = n_elite;
+  if (!all_ties) {         // the first `want` ties by index, behind the candidates below the threshold
+    const int wave = tid >> 6;
+    for (int i0 = 0, seen = 0; seen < want; i0 += kCemThreads) {
+      const int i = i0 + tid;
+      const bool tie = i < n && order_bits(key[i]) == prefix;
+      const unsigned long long in_wave = __ballot(tie);
+      __syncthreads();
+      if (lane == 0) hist[wave] = __popcll(in_wave);
+      __syncthreads();
+      int at = seen + __popcll(in_wave & ((1ULL << lane) - 1));
+      for (int w = 0; w < kCemThreads / 64; ++w) {
+        at += w < wave ? hist[w] : 0;
+        seen += hist[w];
+      }
+      if (tie && at < want) list[m - want + at] = entry(prefix, i);
     }
   }
-  __syncthreads();
-  const int m = count_s;
-  if (m > kListMax) return false;
-  // rank of each against all, the comparisons of one candidate shared by as many threads as there are
-  int* rank = val + kListMax;
   for (int e = tid; e < m; e += kCemThreads) rank[e] = 0;
   __syncthreads();
+  // rank of each against all, the comparisons of one candidate shared by as many threads as there are
   const int parts = m < kCemThreads ? kCemThreads / m : 1;
   for (int t = tid; t < m * parts; t += kCemThreads) {
     const int e = t % m;
@@ -200,14 +215,12 @@ __device__ bool select_elites(const float* key, int* val, unsigned long long* li
     if (parts > 1) atomicAdd(&rank[e], r); else rank[e] = r;
   }
   __syncthreads();
-  for (int e = tid; e < m; e += kCemThreads)
-    if (rank[e] < n_elite) val[rank[e]] = static_cast<int>(list[e] & 0xffffffffu);
+  for (int e = tid; e < m; e += kCemThreads) val[rank[e]] = static_cast<int>(list[e] & 0xffffffffu);
   __syncthreads();
-  return true;
 }
 
 // All (cost, index) pairs sorted ascending in LDS (bitonic network, ties broken by index).
-__device__ void sort_all(float* key, int* val, int n, int npow2) {
+__device__ __forceinline__ void sort_all(float* key, int* val, int n, int npow2) {
   const int tid = threadIdx.x;
   for (int i = tid; i < npow2; i += kCemThreads) {
     float c = i < n ? key[i] : INFINITY;
@@ -232,68 +245,76 @@ __device__ void sort_all(float* key, int* val, int n, int npow2) {
   }
 }
 
-constexpr int kEliteRegs = kSelectMax / 64;
+// Selecting costs eight barriers and a ranking of n_elite^2 comparisons, sorting a barrier per stage of
+// all n (us, selected / sorted): 64 samples with 7 elites 8.4 / 7.9, 100 with 10 8.5 / 9.2, 4096 with
+// 410 21.7 / 73; 512 with 256 11.7 / 15.6 and with 512 17.7 / 16.3; 1000 with 500 18.4 / 22.2 and with
+// 1000 41 / 25; 4096 with 1024 48 / 77.
+__device__ __forceinline__ bool use_selection(int n, int n_elite) {
+  return n_elite <= kSelectMax && n > 64 && 2 * n_elite <= n;
+}
+
+// Mean and sum of squared deviations of a parameter over the elites, one wave: lanes stride over the
+// elites, then a fixed butterfly.  Both passes add the same values in the same order.  R > 0: n_elite
+// <= 64 R, gathered once with all loads in flight; 0: any number, gathered twice.
+template <int R>
+__device__ __forceinline__ float2 elite_moments(const float* __restrict__ th, const int* val, int n_elite, int lane) {
+  float x[R > 0 ? R : 1];
+  float s = 0.0f, v = 0.0f;
+  if (R > 0) {
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+      if (lane + 64 * k < n_elite) x[k] = th[static_cast<unsigned>(val[lane + 64 * k])];
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+      if (lane + 64 * k < n_elite) s += x[k];
+  } else {
+    for (int e = lane; e < n_elite; e += 64) s += th[val[e]];
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+  const float m = s / static_cast<float>(n_elite);
+  if (R > 0) {
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+      if (lane + 64 * k < n_elite) {
+        const float d = x[k] - m;
+        v = fmaf(d, d, v);
+      }
+  } else {
+    for (int e = lane; e < n_elite; e += 64) {
+      const float d = th[val[e]] - m;
+      v = fmaf(d, d, v);
+    }
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  return make_float2(m, v);
+}
 
 // Elites in ascending order of (cost, index), NaN treated as +inf (selected where they are few,
-// else by sorting all), then per-parameter elite moments with wave reductions and the best-so-far.
-// Called by one whole workgroup of kCemThreads threads; keys must already hold the costs.  One
-// workgroup's latency is the time: 4096 samples, 410 elites, 25 parameters 77 -> 32 us.
-__device__ void cem_sort_update(float* key, int* val, unsigned long long* list, int n, int npow2,
+// else by sorting all), then per-parameter elite moments and the best-so-far.  Called by one whole
+// workgroup of kCemThreads threads; keys must already hold the costs.  One workgroup's latency is the
+// time: 4096 samples, 410 elites, 22 parameters 77 us by sorting, 26 us by selecting, 21 us inlined
+// (its LDS and global accesses as such); all costs tied 67, 95 (ties beyond the list were sorted), 20.
+__device__ __forceinline__ void cem_sort_update(float* key, int* val, int n, int npow2,
                                 const float* __restrict__ theta, int ld, int n_param, int n_elite, float alpha,
                                 const float* __restrict__ min_std, float* __restrict__ mean, float* __restrict__ stdv,
                                 float* __restrict__ best, float* __restrict__ best_cost, int* __restrict__ elite_idx) {
   const int tid = threadIdx.x;
-  __shared__ float best_key;
-  if (n_elite <= kSelectMax && select_elites(key, val, list, n, n_elite)) {
-    if (tid == 0) best_key = key[val[0]] == key[val[0]] ? key[val[0]] : INFINITY;
-  } else {
-    __syncthreads();
-    sort_all(key, val, n, npow2);
-    if (tid == 0) best_key = key[0];
-  }
-  __syncthreads();
+  if (use_selection(n, n_elite)) select_elites(key, val, n, n_elite);
+  else sort_all(key, val, n, npow2);            // both end on a barrier; sorted, key[0] is the lowest
+  float best_key = use_selection(n, n_elite) ? key[val[0]] : key[0];
+  if (!(best_key == best_key)) best_key = INFINITY;
   if (elite_idx)
     for (int e = tid; e < n_elite; e += kCemThreads) elite_idx[e] = val[e];
-  // one wave per parameter: lanes stride over the elites, then a fixed butterfly
+  // one wave per parameter
   const int wave = tid / 64, lane = tid % 64, n_waves = kCemThreads / 64;
   for (int p = wave; p < n_param; p += n_waves) {
     const float* th = theta + static_cast<size_t>(p) * ld;
-    // both passes over the same values, in the same order: gathered once, all loads in flight,
-    // where a lane's share fits its registers
-    float x[kEliteRegs];
-    const bool held = n_elite <= kSelectMax;
-    if (held) {
-#pragma unroll
-      for (int k = 0; k < kEliteRegs; ++k)
-        if (lane + 64 * k < n_elite) x[k] = th[val[lane + 64 * k]];
-    }
-    float s = 0.0f;
-    if (held) {
-#pragma unroll
-      for (int k = 0; k < kEliteRegs; ++k)
-        if (lane + 64 * k < n_elite) s += x[k];
-    } else {
-      for (int e = lane; e < n_elite; e += 64) s += th[val[e]];
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    const float m = s / static_cast<float>(n_elite);
-    float v = 0.0f;
-    if (held) {
-#pragma unroll
-      for (int k = 0; k < kEliteRegs; ++k)
-        if (lane + 64 * k < n_elite) {
-          float d = x[k] - m;
-          v += d * d;
-        }
-    } else {
-      for (int e = lane; e < n_elite; e += 64) {
-        float d = th[val[e]] - m;
-        v += d * d;
-      }
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    const float2 mv = n_elite <= 64 ? elite_moments<1>(th, val, n_elite, lane)
+                      : n_elite <= kSelectMax ? elite_moments<kSelectMax / 64>(th, val, n_elite, lane)
+                                              : elite_moments<0>(th, val, n_elite, lane);
+    const float m = mv.x, v = mv.y;
     if (lane == 0) {
       float sd = sqrtf(v / static_cast<float>(n_elite));
       float nm = alpha * mean[p] + (1.0f - alpha) * m;
@@ -318,11 +339,10 @@ __global__ __launch_bounds__(kCemThreads) void cem_update_kernel(
     float alpha, const float* __restrict__ min_std, float* __restrict__ mean, float* __restrict__ stdv,
     float* __restrict__ best, float* __restrict__ best_cost, int* __restrict__ elite_idx, int npow2) {
   __shared__ float key[SPI_MAX_CEM_SAMPLES];
-  __shared__ int val[SPI_MAX_CEM_SAMPLES];
-  __shared__ unsigned long long list[kListMax];
+  __shared__ __attribute__((aligned(8))) int val[SPI_MAX_CEM_SAMPLES];
   for (int i = threadIdx.x; i < n; i += kCemThreads) key[i] = cost[i];
   __syncthreads();
-  cem_sort_update(key, val, list, n, npow2, theta, ld, n_param, n_elite, alpha, min_std, mean, stdv, best, best_cost,
+  cem_sort_update(key, val, n, npow2, theta, ld, n_param, n_elite, alpha, min_std, mean, stdv, best, best_cost,
                   elite_idx);
 }
 
@@ -348,10 +368,11 @@ __global__ void cem_sample_batch_kernel(const SpiBatchProblem* __restrict__ prob
 
 // Batched: one workgroup per problem; segment reduction (fixed order), sort, moments, best,
 // iteration + 1.
-__global__ __launch_bounds__(kCemThreads) void cem_update_batch_kernel(SpiBatchProblem* __restrict__ probs) {
+// 80 scalar registers, so that two workgroups (eight wavefronts per SIMD) share a CU: 300 problems of
+// 128 samples 23 -> 14 us, 512 of 4096 87 -> 62 us.
+__global__ __launch_bounds__(kCemThreads) __attribute__((amdgpu_num_sgpr(80))) void cem_update_batch_kernel(SpiBatchProblem* __restrict__ probs) {
   __shared__ float key[SPI_MAX_CEM_SAMPLES];
-  __shared__ int val[SPI_MAX_CEM_SAMPLES];
-  __shared__ unsigned long long list[kListMax];
+  __shared__ __attribute__((aligned(8))) int val[SPI_MAX_CEM_SAMPLES];
   SpiBatchProblem& P = probs[blockIdx.x];
   const int n = P.n_samples;
   for (int c = threadIdx.x; c < n; c += kCemThreads) {
@@ -362,7 +383,7 @@ __global__ __launch_bounds__(kCemThreads) void cem_update_batch_kernel(SpiBatchP
   __syncthreads();
   int npow2 = 2;
   while (npow2 < n) npow2 <<= 1;
-  cem_sort_update(key, val, list, n, npow2, P.theta, n, SPI_P_COUNT, P.n_elite, P.alpha, P.min_std, P.mean, P.std,
+  cem_sort_update(key, val, n, npow2, P.theta, n, SPI_P_COUNT, P.n_elite, P.alpha, P.min_std, P.mean, P.std,
                   P.best, P.best_cost, nullptr);
   if (threadIdx.x == 0) P.iteration = P.iteration + 1u;
 }

@@ -19,11 +19,14 @@ def _costs(rng, n, kind):
         c[rng.random(n) < 0.1] = np.nan
         c[rng.random(n) < 0.1] = -0.0
         c[rng.random(n) < 0.1] = 0.0
+    elif kind == "mostly diverged":
+        c[rng.random(n) < 0.97] = np.inf
     return c
 
 
-@pytest.mark.parametrize("kind", ["smooth", "ties", "one value", "special"])
-@pytest.mark.parametrize("n,elites", [(1, 1), (65, 65), (1000, 100), (4096, 410), (8192, 820), (8192, 1024), (8191, 1025)])
+@pytest.mark.parametrize("kind", ["smooth", "ties", "one value", "special", "mostly diverged"])
+@pytest.mark.parametrize("n,elites", [(1, 1), (65, 65), (1000, 100), (4096, 410), (8192, 820), (8192, 1024), (8191, 1025),
+                                      (64, 32), (65, 32), (128, 64), (128, 65), (2048, 1024), (2049, 1), (8192, 1)])
 def test_selection_matches_numpy(gpu, n, elites, kind):
     import torch
     from spi_amd import _lib
@@ -47,3 +50,29 @@ def test_selection_matches_numpy(gpu, n, elites, kind):
     assert np.allclose(std.cpu().numpy(), el.std(1), atol=3e-6)
     if np.isfinite(key[want[0]]):
         assert float(best_cost) == key[want[0]] and np.array_equal(best.cpu().numpy(), theta[:, want[0]])
+
+
+def test_tied_costs_take_no_longer(gpu):
+    """A population whose costs all tie (every rollout diverged) or mostly do, against distinct costs."""
+    import torch
+    from spi_amd.agents.cem import CEMConfig, DeviceCEM
+    one = np.ones(22)
+
+    def time(cost):
+        cem = DeviceCEM(0 * one, one, -3 * one, 3 * one, 0.01 * one, CEMConfig(n_samples=4096))
+        cem.ask()
+        c = torch.from_numpy(cost).to(gpu)
+        out = []
+        for _ in range(8):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(20):
+                cem.tell(c)
+            b.record()
+            b.synchronize()
+            out.append(a.elapsed_time(b))
+        return min(out)
+
+    smooth = time(_costs(np.random.default_rng(0), 4096, "smooth"))
+    for kind in ("one value", "mostly diverged", "ties"):
+        assert time(_costs(np.random.default_rng(0), 4096, kind)) < 2 * smooth
