@@ -104,3 +104,32 @@ def test_autotune_keeps_philox_position(gpu, sim, theta0):
     for x, y in zip(ra, rb):
         # same samples; costs may differ in the last bits between launch shapes
         assert np.allclose(x["mean"], y["mean"], rtol=1e-4, atol=1e-6)
+
+
+def test_short_queue_uses_every_cu(gpu, sim, theta0):
+    """256 tasks, one per CU: the batched launch takes no longer than the single launch of the same
+    rollouts, give or take (workgroups beyond the tasks would share the first CUs)."""
+    import torch
+    from spi_amd.agents.batch import BatchCEM, ProblemSpec
+    from spi_amd.agents.sysid import identification_prior
+    from spi_amd.data import synthetic_segments
+    from spi_amd.rollout import RolloutEngine
+    eng = RolloutEngine(sim)
+    segs = eng.upload_segments(synthetic_segments(eng.simulate_np, theta0, sim, n_seg=16, horizon=10, seed=0))
+    batch = BatchCEM(eng, [ProblemSpec(segs, 10, identification_prior(), n_samples=4096)])
+    batch.sample()
+    theta = batch.bufs[0].theta
+
+    def time(f):
+        out = []
+        for _ in range(7):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            f()
+            b.record()
+            b.synchronize()
+            out.append(a.elapsed_time(b))
+        return min(out[2:])
+
+    single = time(lambda: eng.segment_costs(theta, 4096, segs, 10, physics="lanes"))
+    assert batch.n_tasks == 256 and time(batch.rollout) < 1.3 * single
