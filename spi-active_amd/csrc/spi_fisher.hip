@@ -123,10 +123,14 @@ __global__ __launch_bounds__(256) void fim_assemble_vec_kernel(const float* __re
 }
 
 // One workgroup per set: FP64 mean of the valid groups' F, + reg I, Cholesky, logdet.  A thread per
-// entry adds the groups in order, 16 loads in flight; the Cholesky takes a column at a time, a
-// thread per row, each inner product in the order of a serial loop.  512 groups of 22 x 22 in each
-// of 16 sets: 424 us with one load at a time and one thread's Cholesky, 44 us now.
+// entry adds the groups in order, 16 loads in flight; the Cholesky is the first wavefront's, a column
+// at a time, a thread per row, each inner product in the order of a serial loop.  512 groups of 22 x 22
+// in each of 16 sets: 424 us with one load at a time and one thread's Cholesky, 44 us now.  The
+// workgroup is as large as the matrix has entries: with many small sets its idle wavefronts and a
+// Cholesky that all of them went through were the time (4096 sets of 33 groups of 4 x 4 29 us, 46 us
+// with 512 threads each, 14 us now; 4096 sets of 8 of 22 x 22 224, 191, 81).
 constexpr int kLogdetThreads = 512, kLogdetAhead = 16;
+static_assert(SPI_MAX_TANGENTS <= 64, "a wavefront holds a thread per row");
 __global__ __launch_bounds__(kLogdetThreads) void fim_logdet_kernel(const float* __restrict__ F, const int* __restrict__ status,
                                                                     int set_size, int P, const double* __restrict__ scale,
                                                                     double reg, double* __restrict__ Fmean,
@@ -134,16 +138,17 @@ __global__ __launch_bounds__(kLogdetThreads) void fim_logdet_kernel(const float*
   __shared__ double M[SPI_MAX_TANGENTS * SPI_MAX_TANGENTS];
   __shared__ int cnt;
   __shared__ double pivot;
-  const int s = blockIdx.x, tid = threadIdx.x;
+  const int s = blockIdx.x, tid = threadIdx.x, n_threads = blockDim.x;
   const size_t g0 = static_cast<size_t>(s) * set_size;
   if (tid == 0) cnt = 0;
   __syncthreads();
   int mine = 0;
-  for (int c = tid; c < set_size; c += kLogdetThreads) mine += status[g0 + c] == 0;
+#pragma unroll 4
+  for (int c = tid; c < set_size; c += n_threads) mine += status[g0 + c] == 0;
   if (mine) atomicAdd(&cnt, mine);
   __syncthreads();
   const int n = cnt, PP = P * P;
-  for (int e = tid; e < PP; e += kLogdetThreads) {
+  for (int e = tid; e < PP; e += n_threads) {
     const float* f = F + g0 * PP + e;
     const int* st = status + g0;
     double acc = 0.0;
@@ -177,31 +182,31 @@ __global__ __launch_bounds__(kLogdetThreads) void fim_logdet_kernel(const float*
   if (tid < P) M[tid * P + tid] += pivot;
   __syncthreads();
   if (Fmean)
-    for (int e = tid; e < PP; e += kLogdetThreads) Fmean[static_cast<size_t>(s) * PP + e] = M[e];
+    for (int e = tid; e < PP; e += n_threads) Fmean[static_cast<size_t>(s) * PP + e] = M[e];
   __syncthreads();
-  // symmetric part, then in-place Cholesky (lower) in FP64
+  if (tid >= 64) return;
+  // symmetric part, then in-place Cholesky (lower) in FP64, one wavefront
   double ld = 0.0;
   bool pd = n > 0;
   for (int j = 0; j < P && pd; ++j) {
+    double d = 0.0;
     if (tid == j) {
-      double d = M[j * P + j];
+      d = M[j * P + j];
       for (int k = 0; k < j; ++k) d -= M[j * P + k] * M[j * P + k];
-      pivot = d;
     }
-    __syncthreads();
-    const double d = pivot;
+    d = __shfl(d, j, 64);
     pd = d > 0.0;
     if (pd) {
       const double ljj = sqrt(d);
       ld += 2.0 * log(ljj);
-      if (tid == j) M[j * P + j] = ljj;
       if (tid > j && tid < P) {
         double v = 0.5 * (M[tid * P + j] + M[j * P + tid]);
         for (int k = 0; k < j; ++k) v -= M[tid * P + k] * M[j * P + k];
         M[tid * P + j] = v / ljj;
       }
     }
-    __syncthreads();
+    __threadfence_block();                // this column, before the rows that read it
+    __builtin_amdgcn_wave_barrier();
   }
   if (tid == 0) {
     logdet[s] = pd ? ld : -INFINITY;
@@ -331,7 +336,8 @@ int spi_fim_logdet(const float* F_dev, const int* status_dev, int n_sets, int se
       !status_dev || !logdet_dev || !n_valid_dev)
     return ffail(SPI_ERR_INVALID_ARG, "spi_fim_logdet: bad arguments");
   if (n_sets == 0) return SPI_OK;
-  fim_logdet_kernel<<<n_sets, kLogdetThreads, 0, stream>>>(F_dev, status_dev, set_size, n_tan, scale_dev, reg, F_mean_dev,
+  const int threads = n_tan * n_tan <= 64 ? 64 : n_tan * n_tan <= 256 ? 256 : kLogdetThreads;
+  fim_logdet_kernel<<<n_sets, threads, 0, stream>>>(F_dev, status_dev, set_size, n_tan, scale_dev, reg, F_mean_dev,
                                                 logdet_dev, n_valid_dev);
   return flaunch("fim_logdet_kernel");
 }
