@@ -101,8 +101,10 @@ __device__ __forceinline__ int sampled_slot(const SpiCommandSpec& c, int k) {
 // A workgroup takes 256 consecutive steps of up to `per` consecutive trials: a thread forms its
 // step's basis once for all of them, each trial's sampled commands go through LDS, and its run of
 // 256 n_dims output words is written in float4 (VEC: n_dims and the steps of a trial make every
-// run a multiple of 16 bytes).  Bound by the output: 1024 trials x 1250 steps x 14 (71.7 MB) in
-// 26 us; 45 us with a basis per (trial, step) and all 14 commands through LDS.
+// run a multiple of 16 bytes; word by word otherwise).  Bound by the output: 1024 Bezier trials x 1250
+// steps x 14 (71.7 MB) in 26 us; 45 us with a basis per (trial, step) and all 14 commands through LDS.
+// The streaming stores hold for small outputs too: with a kernel that reads all of it behind, 16, 128
+// and 1024 trials of 1250 steps 11.4 -> 9.6, 19.8 -> 17.7 and 68 -> 50 us.
 typedef float FloatX4 __attribute__((ext_vector_type(4)));
 constexpr int kStepThreads = 256, kTrialsPerBlock = 8;
 template <bool VEC>
@@ -121,42 +123,38 @@ __global__ __launch_bounds__(kStepThreads) void command_trials_kernel(SpiCommand
   }
   const StepBasis sb = step_basis(c, min(step, T - 1));
   const int b0 = blockIdx.y * per, b1 = min(b0 + per, n_trials);
-  // step and dimension of this thread's first float4, and what 256 float4 further adds
-  const int sv = 4 * tid / nd, kv = 4 * tid - sv * nd, ds = 4 * kStepThreads / nd, dk = 4 * kStepThreads - ds * nd;
+  // step and dimension of this thread's first W words, and what 256 of these further adds
+  constexpr int W = VEC ? 4 : 1;
+  const int sv = W * tid / nd, kv = W * tid - sv * nd, ds = W * kStepThreads / nd, dk = W * kStepThreads - ds * nd;
   for (int b = b0; b < b1; ++b) {
     const float* p = params + static_cast<size_t>(b) * n_params;
     for (int d = 0; d < c.n_sampled; ++d) val[d * kStepThreads + tid] = sampled_command(c, sb, p, d, c.sampled_idx[d]);
     __syncthreads();
     float* o = out + (static_cast<size_t>(b) * T + static_cast<size_t>(blockIdx.x) * kStepThreads) * nd;
     const int n_out = n_steps * nd;
-    if (VEC) {
-      FloatX4* o4 = reinterpret_cast<FloatX4*>(o);
-      int s0 = sv, k0 = kv;
-      for (int e = tid; 4 * e < n_out; e += kStepThreads) {
-        float v[4];
-        int s = s0, k = k0;
+    int s0 = sv, k0 = kv;
+    for (int e = tid; W * e < n_out; e += kStepThreads) {
+      float v[W];
+      int s = s0, k = k0;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int2 a = at[k];
-          v[q] = val[a.x + a.y * s];
-          if (++k == nd) { k = 0; ++s; }
-        }
-        __builtin_nontemporal_store(FloatX4{v[0], v[1], v[2], v[3]}, o4 + e);   // written once, not read here
-        s0 += ds;
-        k0 += dk;
-        if (k0 >= nd) { k0 -= nd; ++s0; }
+      for (int q = 0; q < W; ++q) {
+        const int2 a = at[k];
+        v[q] = val[a.x + a.y * s];
+        if (++k == nd) { k = 0; ++s; }
       }
-    } else {
-      for (int e = tid; e < n_out; e += kStepThreads) {
-        const int s = e / nd, k = e - s * nd;
-        o[e] = val[at[k].x + at[k].y * s];
-      }
+      if constexpr (VEC)    // written once, not read here
+        __builtin_nontemporal_store(FloatX4{v[0], v[1], v[2], v[3]}, reinterpret_cast<FloatX4*>(o) + e);
+      else
+        o[e] = v[0];
+      s0 += ds;
+      k0 += dk;
+      if (k0 >= nd) { k0 -= nd; ++s0; }
     }
     __syncthreads();
   }
 }
 
-// Trials shorter than a workgroup: one thread per (trial, step) over the flat run of all trials, its
+// Short trials, constants: one thread per (trial, step) over the flat run of all trials, its
 // commands staged in LDS; the workgroup's 256 steps are one
 // contiguous run of the output, written back with consecutive threads on consecutive words.
 // Idx: int while the launch has fewer than 2^31 (trial, step) pairs, long long above.
@@ -172,10 +170,10 @@ __global__ __launch_bounds__(256) void command_kernel(SpiCommandSpec c, const fl
     const int b = static_cast<int>(idx / T);
     const StepBasis sb = step_basis(c, static_cast<int>(idx - static_cast<Idx>(b) * T));
     const float* p = params + static_cast<size_t>(b) * n_params;
-    for (int k = 0; k < c.n_dims; ++k) {
-      const int d = sampled_slot(c, k);
-      stage[threadIdx.x * c.n_dims + k] = d >= 0 ? sampled_command(c, sb, p, d, k) : c.default_cmd[k];
-    }
+    float* o = stage + threadIdx.x * c.n_dims;
+    for (int k = 0; k < c.n_dims; ++k) o[k] = c.default_cmd[k];
+    for (int d = 0; d < c.n_sampled; ++d)      // the last listed wins, as in sampled_slot
+      o[c.sampled_idx[d]] = sampled_command(c, sb, p, d, c.sampled_idx[d]);
   }
   __syncthreads();
   const Idx left = pairs - base;
@@ -205,8 +203,18 @@ int spi_command_sequences(const SpiCommandSpec* spec, const float* params_dev, i
   const long long pairs = static_cast<long long>(n_trials) * spec->n_updates * spec->steps_per_update;
   if (pairs == 0) return SPI_OK;
   const long long T = static_cast<long long>(spec->n_updates) * spec->steps_per_update;
-  // from three quarters of a workgroup's steps on, a workgroup per trial's steps keeps its threads busy
-  if (T >= 192 && T <= 0x7fffffffLL - kStepThreads) {
+  // A workgroup per 256 steps of some trials where the basis that these share costs more than the part of
+  // the last workgroup that stands idle (4096 trials x 14, us against the flat run): Bezier from 192
+  // steps on (195 steps 24.7 / 29.4, 260 32.3 / 35.1, 1250 81 / 142), polynomials with at least two
+  // thirds of the threads at work (200 19.2 / 21.4, 520 36.6 / 45.6, 625 47.8 / 55.7; but 265 39.4 / 26.4,
+  // 300 32.0 / 29.4), constants, which have no basis, for the wide stores of one workgroup per trial (200
+  // 11.4 / 12.6; but 255 15.4 / 14.1, 1250 72 / 50).
+  const bool vec = (T * spec->n_dims) % 4 == 0 && reinterpret_cast<uintptr_t>(out_dev) % 16 == 0;
+  const long long gx256 = (T + kStepThreads - 1) / kStepThreads * kStepThreads;
+  const bool by_trial = T >= 192 && (spec->mode == SPI_COMMAND_BEZIER ? true
+                                     : spec->mode == SPI_COMMAND_POLYNOMIAL ? 3 * T >= 2 * gx256
+                                                                            : vec && T <= kStepThreads);
+  if (by_trial && T <= 0x7fffffffLL - kStepThreads) {
     const unsigned gx = static_cast<unsigned>((T + kStepThreads - 1) / kStepThreads);
     // enough trials per workgroup to share a basis, few enough to leave four workgroups per CU
     const long long groups = static_cast<long long>(gx) * n_trials;
@@ -214,7 +222,6 @@ int spi_command_sequences(const SpiCommandSpec* spec, const float* params_dev, i
     if (per < 1) per = 1;
     while ((n_trials + per - 1) / per > 65535) per *= 2;
     const dim3 grid(gx, static_cast<unsigned>((n_trials + per - 1) / per));
-    const bool vec = (T * spec->n_dims) % 4 == 0 && reinterpret_cast<uintptr_t>(out_dev) % 16 == 0;
     const int Ti = static_cast<int>(T);
     if (vec) command_trials_kernel<true><<<grid, kStepThreads, 0, stream>>>(*spec, params_dev, n_trials, n_params, Ti, per, out_dev);
     else command_trials_kernel<false><<<grid, kStepThreads, 0, stream>>>(*spec, params_dev, n_trials, n_params, Ti, per, out_dev);

@@ -34,7 +34,8 @@ def test_store_windows_equal_the_rows(gpu, lengths, horizon):
 
 
 @pytest.mark.parametrize("mode", ["constant", "polynomial", "bezier"])
-@pytest.mark.parametrize("trials,steps,width", [(1, 38, 14), (33, 39, 13), (5, 51, 14), (1, 52, 13), (2100, 50, 13), (3, 250, 11)])
+@pytest.mark.parametrize("trials,steps,width", [(1, 38, 14), (33, 39, 13), (5, 51, 14), (1, 52, 13), (2100, 50, 13), (3, 250, 11),
+                                                (2100, 53, 14), (40, 76, 13), (40, 77, 13), (9, 125, 11)])
 def test_command_sequences_at_edges(gpu, mode, trials, steps, width):
     import torch
     import spio_commands as oc
@@ -50,3 +51,26 @@ def test_command_sequences_at_edges(gpu, mode, trials, steps, width):
     for k in sorted({0, trials // 2, trials - 1}):
         ref = oc.commands_from_params(P[k], mode, RANGES[:width], DEFAULT[:width], IDX, U, S)
         assert np.abs(out[k] - ref).max() < 2e-6
+
+
+def test_command_time_is_even_over_the_steps(gpu):
+    """A few steps past 256 do not cost a second workgroup per trial."""
+    import torch
+    from spi_amd.agents.commands import CommandGenerator
+    from test_commands_oracle import DEFAULT, IDX, RANGES
+
+    def time(steps):
+        gen = CommandGenerator(RANGES, DEFAULT, IDX, "polynomial", rollout_length=5.0, horizon_length=1.0, dt=1.0 / steps)
+        p = torch.rand((4096, len(gen.param_names())), device=gpu)
+        out = []
+        for _ in range(9):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(20):
+                gen.generate(p)
+            b.record()
+            b.synchronize()
+            out.append(a.elapsed_time(b))
+        return min(out)
+
+    assert time(53) < 1.35 * time(51)
