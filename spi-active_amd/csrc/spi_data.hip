@@ -50,10 +50,14 @@ __device__ __forceinline__ float record_elem(const float* states, const float* a
 // records are one run of the output, written in float4.  A group is staged when its windows'
 // rows lie within `cap` rows of its first one (consecutive windows share all rows but one; a
 // group across the end of a trajectory has a gap of H); otherwise each element is read from the
-// buffers.  A window whose rows r .. r + H do not all lie below n_rows is written as NaN and
+// buffers: short records in one run over the group (5000 random rows, H 1 23 us by window, which
+// leaves two thirds of the threads idle, 9 us so), long ones by window (H 400 1,118 us in one run,
+// 1,066 by window, its row in a scalar register).  A single short window is not worth staging (H 1 2.8 ->
+// 2.4 us).  A window whose rows r .. r + H do not all lie below n_rows is written as NaN and
 // nothing outside the buffers is read.  Bound by the output: 64 x 2500 steps, H 20 (646 MB) in
-// 147 us; 232 us with a division per element, word stores and groups across trajectories
+// 151 us; 232 us with a division per element, word stores and groups across trajectories
 // read element by element.
+constexpr int kShortRecord = 1024;
 template <class Rows>
 __global__ __launch_bounds__(256) void pack_windows_kernel(const float* __restrict__ states,
                                                            const float* __restrict__ actions, Rows rows, int n_rows,
@@ -66,7 +70,7 @@ __global__ __launch_bounds__(256) void pack_windows_kernel(const float* __restri
   const int r0 = rows(w0, H);
   const int rj = tid < nw ? rows(w0 + tid, H) : r0;
   if (tid == 0) last = 0;
-  const bool near = rj >= 0 && r0 >= 0 && rj >= r0 && static_cast<long long>(rj) - r0 + H < cap &&
+  const bool near = (nw > 1 || stride > kShortRecord) && rj >= 0 && r0 >= 0 && rj >= r0 && static_cast<long long>(rj) - r0 + H < cap &&
                     static_cast<long long>(rj) + H < n_rows;
   const bool staged = __syncthreads_and(near);
   float* o = out + static_cast<size_t>(w0) * stride;
@@ -121,11 +125,25 @@ __global__ __launch_bounds__(256) void pack_windows_kernel(const float* __restri
     }
     return;
   }
-  for (int w = 0; w < nw; ++w) {
-    const int t = rows(w0 + w, H);
-    const bool ok = t >= 0 && static_cast<long long>(t) + H < n_rows;
-    for (int e = tid; e < stride; e += 256)
-      o[static_cast<size_t>(w) * stride + e] = ok ? record_elem(states, actions, t, e) : __int_as_float(0x7fc00000);
+  if (stride > kShortRecord) {
+    for (int w = 0; w < nw; ++w) {
+      const int t = rows(w0 + w, H);
+      const bool ok = t >= 0 && static_cast<long long>(t) + H < n_rows;
+      for (int e = tid; e < stride; e += 256)
+        o[static_cast<size_t>(w) * stride + e] = ok ? record_elem(states, actions, t, e) : __int_as_float(0x7fc00000);
+    }
+    return;
+  }
+  if (tid < nw) at[tid] = rj >= 0 && static_cast<long long>(rj) + H < n_rows ? rj : -1;
+  __syncthreads();
+  const int n_out = nw * stride, qw = 256 / stride, qe = 256 - qw * stride;
+  int w = tid / stride, e = tid - w * stride;
+  for (int f = tid; f < n_out; f += 256) {
+    const int t = at[w];
+    o[f] = t >= 0 ? record_elem(states, actions, t, e) : __int_as_float(0x7fc00000);
+    w += qw;
+    e += qe;
+    if (e >= stride) { e -= stride; ++w; }
   }
 }
 

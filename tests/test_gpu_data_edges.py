@@ -33,6 +33,54 @@ def test_store_windows_equal_the_rows(gpu, lengths, horizon):
         assert np.array_equal(b.kp, 20.0 + np.array(src)) and np.array_equal(b.kd, np.float32(0.5) + np.array(src))
 
 
+@pytest.mark.parametrize("horizon", [1, 4, 5, 20, 21, 330])     # 20: the longest short record
+@pytest.mark.parametrize("n", [1, 2, 3, 65, 130])
+@pytest.mark.parametrize("order", ["run", "random", "reversed"])
+def test_row_tables_equal_the_rows(gpu, horizon, n, order):
+    """Windows of any rows, rows outside the buffer (NaN records) among them."""
+    import torch
+    from spi_amd import _lib
+    rng = np.random.default_rng(horizon + n)
+    R = 500
+    s, a = rng.normal(size=(R, 37)).astype(np.float32), rng.normal(size=(R, 12)).astype(np.float32)
+    rows = {"run": 7 + np.arange(n), "random": rng.integers(-3, R, n), "reversed": R - 1 - np.arange(n)}[order].astype(np.int32)
+    d = lambda x: torch.from_numpy(x).to(gpu)
+    sd, ad, rd = d(s), d(a), d(rows)
+    out = torch.empty((n, 37 + 49 * horizon), device=gpu)
+    _lib.check(_lib.lib().spi_pack_windows_rows(_lib.ptr(sd), _lib.ptr(ad), R, _lib.ptr(rd, torch.int32), n, horizon,
+                                                _lib.ptr(out), _lib.stream()), "spi_pack_windows_rows")
+    out = out.cpu().numpy()
+    for w, r in enumerate(rows):
+        if r < 0 or r + horizon >= R:
+            assert np.isnan(out[w]).all()
+        else:
+            rec = np.concatenate([a[r:r + horizon], s[r + 1:r + horizon + 1]], 1).reshape(-1)
+            assert np.array_equal(out[w], np.concatenate([s[r], rec]))
+
+
+def test_short_records_of_scattered_rows_take_no_longer(gpu):
+    """Rows in any order read element by element: one-step records within a few times consecutive rows'."""
+    import torch
+    from spi_amd import _lib
+    R, n = 20000, 5000
+    s, a, out = torch.randn((R, 37), device=gpu), torch.randn((R, 12), device=gpu), torch.empty((n, 86), device=gpu)
+
+    def time(rows):
+        rd, best = torch.from_numpy(rows.astype(np.int32)).to(gpu), []
+        for _ in range(9):
+            t0, t1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            t0.record()
+            for _ in range(20):
+                _lib.check(_lib.lib().spi_pack_windows_rows(_lib.ptr(s), _lib.ptr(a), R, _lib.ptr(rd, torch.int32), n, 1,
+                                                            _lib.ptr(out), _lib.stream()), "spi_pack_windows_rows")
+            t1.record()
+            t1.synchronize()
+            best.append(t0.elapsed_time(t1))
+        return min(best)
+
+    assert time(np.arange(n)[::-1]) < 1.7 * time(np.arange(n))
+
+
 @pytest.mark.parametrize("mode", ["constant", "polynomial", "bezier"])
 @pytest.mark.parametrize("trials,steps,width", [(1, 38, 14), (33, 39, 13), (5, 51, 14), (1, 52, 13), (2100, 50, 13), (3, 250, 11),
                                                 (2100, 53, 14), (40, 76, 13), (40, 77, 13), (9, 125, 11)])
