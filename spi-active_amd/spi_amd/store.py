@@ -63,26 +63,26 @@ class SegmentStore:
         self._joined = None
 
     def _joined_buffers(self):
-        return self._joined_with_rows()[:3]
+        return self._joined_with_rows(_lib.stream())[:3]
 
-    def _joined_with_rows(self):
+    def _joined_with_rows(self, stream: int):
         """All trajectories back to back in one device buffer (rebuilt after an add).  A later call
         may run on any stream and cannot order itself after a build that it does not know of, so
         the build is complete before its buffers are kept; a call on another stream than the
-        build's marks them as used there, so that a rebuild does not hand their memory on early."""
-        stream = torch.cuda.current_stream(self.device)
+        build's marks them as used there, so that a rebuild does not hand their memory on early.
+        stream: handle of the current stream."""
         joined = self._joined
         if joined is None or len(joined[0][2]) != len(self.trajectories):
             trs = list(self.trajectories)
             starts = np.cumsum([0] + [tr.n_steps for tr in trs])[:-1]
             kept = (torch.cat([tr.states for tr in trs]), torch.cat([tr.actions for tr in trs]), starts,
                     torch.from_numpy(np.minimum(starts, 2 ** 31 - 1).astype(np.int32)).to(self.device))
-            stream.synchronize()
+            torch.cuda.current_stream().synchronize()
             self._joined = joined = (kept, stream)
         kept, built_on = joined
         if stream != built_on:
             for t in (kept[0], kept[1], kept[3]):
-                t.record_stream(stream)
+                t.record_stream(torch.cuda.current_stream())
         return kept
 
     def add_arrays(self, states: np.ndarray, actions: np.ndarray, kp: float = 20.0, kd: float = 0.5,
@@ -112,7 +112,8 @@ class SegmentStore:
         if n == 0:
             raise ValueError("no trajectory is longer than the horizon")
         out = torch.empty((n, segment_stride(horizon)), dtype=torch.float32, device=self.device)
-        states, actions, first, first_dev = self._joined_with_rows()
+        stream = _lib.stream()
+        states, actions, first, first_dev = self._joined_with_rows(stream)
         if states.shape[0] >= 2 ** 31:
             raise ValueError("the store holds more than 2^31 - 1 trajectory rows")
         # every window of every trajectory: the kernel finds the rows itself; a choice of
@@ -129,7 +130,7 @@ class SegmentStore:
         if whole:
             rc = L.spi_pack_windows_store(_lib.ptr(states), _lib.ptr(actions), states.shape[0],
                                           _lib.ptr(first_dev, torch.int32), len(which), n, horizon, _lib.ptr(out),
-                                          _lib.stream())
+                                          stream)
             _lib.check(rc, "spi_pack_windows_store")
         L.spi_window_index(len(which), *[a.ctypes.data for a in table], ends.ctypes.data, src.ctypes.data,
                            start.ctypes.data, kp.ctypes.data, kd.ctypes.data, None if whole else rows.ctypes.data)
@@ -137,6 +138,6 @@ class SegmentStore:
             return SegmentBatch(out, horizon, ends, src, start, kp, kd)
         rows_dev = torch.from_numpy(rows).to(self.device)
         rc = L.spi_pack_windows_rows(_lib.ptr(states), _lib.ptr(actions), states.shape[0],
-                                     _lib.ptr(rows_dev, torch.int32), n, horizon, _lib.ptr(out), _lib.stream())
+                                     _lib.ptr(rows_dev, torch.int32), n, horizon, _lib.ptr(out), stream)
         _lib.check(rc, "spi_pack_windows_rows")
         return SegmentBatch(out, horizon, ends, src, start, kp, kd)

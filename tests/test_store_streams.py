@@ -6,7 +6,7 @@ import pytest
 
 class _Stream:
     def __init__(self, log, name):
-        self.log, self.name = log, name
+        self.log, self.name, self.cuda_stream = log, name, ord(name)
 
     def synchronize(self):
         self.log.append("synchronize " + self.name)
