@@ -546,8 +546,10 @@ int spi_rollout_cost(const SpiSimArgs* sim, const SpiCostArgs* cost, const float
     return fail(SPI_ERR_INVALID_ARG, "spi_rollout_cost: bad sizes or null pointer");
   if (n_cand == 0 || n_seg == 0) return SPI_OK;
   const int stride = spi_segment_stride(horizon);
-  const size_t lds_bytes = static_cast<size_t>(stride) * sizeof(float);
-  if (lds_bytes > 64 * 1024) return fail(SPI_ERR_TOO_LARGE, "spi_rollout_cost: horizon too long for LDS staging");
+  // the four-lane kernel's limit, which stages a record in LDS: the horizons that are taken do not
+  // depend on the size of a batch
+  const size_t record_bytes = static_cast<size_t>(stride) * sizeof(float);
+  if (record_bytes > 64 * 1024) return fail(SPI_ERR_TOO_LARGE, "spi_rollout_cost: record over 64 KB (horizon over 333)");
   const int n_cblk = (n_cand + kRolloutThreads - 1) / kRolloutThreads;
   const long long nblk = static_cast<long long>(n_cblk) * n_seg;
   if (nblk > 0x7fffffffLL || static_cast<long long>(n_seg) * n_cand > (1LL << 31))
@@ -567,7 +569,7 @@ int spi_rollout_cost_legs(const SpiSimArgs* sim, const SpiCostArgs* cost, const 
   if (n_cand == 0 || n_seg == 0) return SPI_OK;
   const int stride = spi_segment_stride(horizon);
   const size_t lds_bytes = static_cast<size_t>(stride) * sizeof(float);
-  if (lds_bytes > 64 * 1024) return fail(SPI_ERR_TOO_LARGE, "spi_rollout_cost_legs: horizon too long for LDS staging");
+  if (lds_bytes > 64 * 1024) return fail(SPI_ERR_TOO_LARGE, "spi_rollout_cost_legs: record over 64 KB of LDS (horizon over 333)");
   const int per_block = kRolloutThreads / 4;
   const int n_cblk = (n_cand + per_block - 1) / per_block;
   const long long nblk = static_cast<long long>(n_cblk) * n_seg;
@@ -606,8 +608,8 @@ int spi_batch_rollout_cost(const SpiSimArgs* sim, const SpiBatchProblem* probs_d
   if (n_prob < 1 || n_tasks < 0 || max_horizon < 1 || n_blocks < 1 || !probs_dev || !task_prefix_dev || !queue_dev)
     return fail(SPI_ERR_INVALID_ARG, "spi_batch_rollout_cost: bad arguments");
   if (n_tasks == 0) return SPI_OK;
-  const size_t lds = static_cast<size_t>(spi_segment_stride(max_horizon)) * sizeof(float);
-  if (lds > 64 * 1024) return fail(SPI_ERR_TOO_LARGE, "spi_batch_rollout_cost: horizon too long for LDS staging");
+  const size_t record_bytes = static_cast<size_t>(spi_segment_stride(max_horizon)) * sizeof(float);   // as spi_rollout_cost
+  if (record_bytes > 64 * 1024) return fail(SPI_ERR_TOO_LARGE, "spi_batch_rollout_cost: record over 64 KB (horizon over 333)");
   // No more workgroups than tasks: a CU holds two, and those of the CUs filled first would take all of a
   // short queue while the other CUs stand idle (4096 candidates x 16 segments x H 20, 256 tasks: 2,330 ->
   // 1,380 us).

@@ -322,7 +322,7 @@ def test_derivative_entry_points_reject_bad_arguments():
 
 def test_empty_inputs_return_ok_and_oversized_are_refused():
     """Zero candidates / segments / samples / excitations return SPI_OK without touching the
-    device (the calls run here, with no GPU); records that do not fit the 64 KB LDS staging
+    device (the calls run here, with no GPU); records over the 64 KB that the four-lane kernel stages
     (horizon 400 for segments, 1400 for excitations) and CEM updates of more than
     SPI_MAX_CEM_SAMPLES samples are refused on the host."""
     import torch  # noqa: F401
