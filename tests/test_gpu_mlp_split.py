@@ -1,6 +1,6 @@
 """The actor's layers on split products at the edges of their tiles: row counts around a tile, widths
-that leave part of one, inputs of three magnitudes, and non-finite inputs, against float64 and
-against plain float32 products."""
+that leave part of one, inputs of three magnitudes, of few non-zero values, of one sign and from either
+end of the range, and non-finite inputs in every tile shape, dense and from a ring, against float64."""
 import numpy as np
 import pytest
 
@@ -46,6 +46,8 @@ def test_non_finite_inputs_stay_in_their_row(gpu):
     keep = [i for i in range(130) if i not in (5, 70, 129)]
     assert np.array_equal(got[keep], clean[keep])
     assert np.isnan(got[70]).all() and not np.isfinite(got[5]).any()
+    want = _f64(net, bad[129:])[0]                       # 1e37 per unit, 1e36 per output
+    assert np.abs(want).max() < 3e38 and np.abs(got[129] - want).max() <= 5e-6 * np.abs(want).max()
     # one hidden layer of an infinite input: each unit is its weight's sign times infinity
     one = _net((64, 64), 1)
     y = np.zeros((1, 64), np.float32)
@@ -144,6 +146,7 @@ def test_non_finite_and_huge_operands_in_every_tile_shape(gpu, rows, width, ring
         return net.forward_ring(buf, 1, kmap, 3.3e38, rows, row0=ring).cpu().numpy()
 
     clean, got = run(x), run(bad)
+    assert np.array_equal(clean, net(torch.from_numpy(x).to(gpu)).cpu().numpy())   # ring and dense: the same bits
     keep = np.setdiff1d(np.arange(rows), list(at))
     assert np.array_equal(got[keep], clean[keep])
     if ring is not None:

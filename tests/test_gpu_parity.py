@@ -114,6 +114,49 @@ def test_physics_step_matches_oracle(gpu, model, sim, theta0):
     assert perr <= 5e-6 and verr <= 1e-3, (perr, verr)
 
 
+def test_physics_step_forms_at_their_line(gpu, model, sim, theta0):
+    """spi_physics_step takes four lanes per env up to 32,768 envs and one above.  128 realistic states
+    and parameter rows, repeated: each form against the oracle, every env of the last workgroup and
+    all others equal to its first copy bit for bit, with and without foot forces; the two forms agree
+    within twice the oracle's bounds."""
+    import torch
+    o, s = _oracle(model, sim)
+    eng = _engine(s)
+    rng = np.random.default_rng(21)
+    m = 128
+    states = _realistic_states(model, s, theta0, m, seed=22)
+    rows, tau = _rand_params(rng, theta0, m), rng.normal(0, 5, (m, 12)).astype(np.float32)
+    ref = [o.physics_step(*(np.split(states[i].astype(np.float32).astype(np.float64), [13, 25])), tau[i],
+                          rows[i].astype(np.float32).astype(np.float64)) for i in range(m)]
+    first = {}
+    for n in (32768, 32769):
+        at = np.arange(n) % m
+        P, t = _soa(rows[at], gpu), torch.from_numpy(tau[at]).to(gpu)
+        out = {}
+        for force in (True, False):
+            root = torch.from_numpy(states[at, :13].astype(np.float32)).to(gpu)
+            dof = torch.from_numpy(np.stack([states[at, 13:25], states[at, 25:37]], 2).astype(np.float32)).to(gpu).contiguous()
+            ff = torch.full((n, 12), -1.0, dtype=torch.float32, device=gpu) if force else None
+            eng.physics_step(P, root, dof, t, ff)
+            out[force] = [x.cpu().numpy() for x in (root, dof, ff) if x is not None]
+        for a, b in zip(out[False], out[True]):
+            assert np.array_equal(a, b)
+        for x in out[True]:
+            assert np.array_equal(x, x[at])
+        first[n] = [x[:m].astype(np.float64) for x in out[True]]
+        root, dof, ff = first[n]
+        pos = max(np.abs(root[i, :7] - r[0][:7]).max() for i, r in enumerate(ref))
+        vel = max(np.abs(root[i, 7:] - r[0][7:]).max() for i, r in enumerate(ref))
+        pos = max(pos, *(np.abs(dof[i, :, 0] - r[1]).max() for i, r in enumerate(ref)))
+        vel = max(vel, *(np.abs(dof[i, :, 1] - r[2]).max() for i, r in enumerate(ref)))
+        print(f"{n} envs: max pos err {pos:.3g}, max vel err {vel:.3g}, in contact {(np.abs(ff).sum(1) > 0).sum()}")
+        assert pos <= 5e-6 and vel <= 1e-3 and (np.abs(ff).sum(1) > 0).sum() > m // 4
+    (ra, da, fa), (rb, db, fb) = first[32768], first[32769]
+    assert np.abs(ra - rb)[:, :7].max() <= 1e-5 and np.abs(ra - rb)[:, 7:].max() <= 2e-3
+    assert np.abs(da - db)[..., 0].max() <= 1e-5 and np.abs(da - db)[..., 1].max() <= 2e-3
+    assert np.abs(fa - fb).max() <= 1.0            # 1e-5 m at 5e4 N/m and 2e-3 m/s at 100 N s/m
+
+
 def test_forward_dynamics_matches_oracle(gpu, model, sim, theta0):
     """Accelerations (base spatial acceleration + qdd) of the specialised FP32 ABA vs the FP64
     generic-tree ABA on realistic states: |da| <= 1e-3 * max|a| per env."""

@@ -57,9 +57,11 @@ def test_host_elimination_matches_oracle(tmp_path, model, sim, theta0, double, m
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,horizon", [(1, 1), (255, 2), (257, 1), (300, 60)])
-def test_rollout_cost_at_edges(gpu, sim, theta0, n, horizon):
-    """One lane per rollout, workgroup edges and a horizon of one step or more than one staging
-    buffer once held: the cost of the recorded truth's neighbours against the record mode."""
+def test_rollout_cost_at_edges(gpu, model, sim, theta0, n, horizon):
+    """One lane per rollout at workgroup edges and a short and a long horizon: every cost against the
+    record mode (which candidate and segment it belongs to; both inline the same step), and up to two
+    steps a sample against the FP64 oracle (its value)."""
+    import spio
     import torch
     from spi_amd.agents.sysid import identification_prior
     from spi_amd.data import synthetic_segments
@@ -80,3 +82,8 @@ def test_rollout_cost_at_edges(gpu, sim, theta0, n, horizon):
         # squared error at the noise floor turns into 1e-3 at most where nothing is chaotic)
         ok = np.abs(got[s] - want) <= 2e-3 * want + 1e-4
         assert ok.mean() > (0.99 if horizon <= 20 else 0.9), np.abs(got[s] / want - 1).max()
+    if horizon <= 2:
+        at = np.unique(np.clip([0, 1, n // 3, 63, n - 2, n - 1], 0, n - 1))
+        ref = spio.Oracle(model, sim).rollout_cost(rows[at].astype(np.float64), segs.init, segs.actions, segs.targets, 0,
+                                                   np.asarray(eng.cargs.w[:], np.float64))
+        assert (np.abs(got[:, at].T - ref) <= 2e-3 * ref + 1e-4).all()
