@@ -188,15 +188,17 @@ int spi_fd_fim_trace(const float* root_dev, const float* dof_state_dev, const fl
 /* ---- fused hot path ---- */
 
 /* Fused rollout + tracking cost: for every (segment s, candidate c) run `horizon` control
- * steps of PD + motor model + ABA + contact + semi-implicit Euler from the segment's initial
+ * steps of PD + motor model + forward dynamics (each leg eliminated in its hip frame) + contact +
+ * semi-implicit Euler from the segment's initial
  * state and write cost_seg_dev[s * n_cand + c].  Replaces the eager loop of
  * scripts/eval.py:239-296 (and the per-candidate Python loop of mass_landscape.py:123-126).
- * seg_dev: [n_seg][spi_segment_stride(horizon)] floats.  Diverged lanes get +inf. */
+ * seg_dev: [n_seg][spi_segment_stride(horizon)] floats, a record at most 64 KB (horizon <= 333, here
+ * and in the four-lane and batched forms).  Diverged lanes get +inf. */
 int spi_rollout_cost(const SpiSimArgs* sim, const SpiCostArgs* cost, const float* params_dev, int ld, int n_cand,
                      const float* seg_dev, int n_seg, int horizon, float* cost_seg_dev, hipStream_t stream);
 
-/* The same costs with four lanes per (candidate, segment), one per leg (base replicated, the
- * legs' articulated inertias summed across the four lanes): lower latency for batches that
+/* The same costs with four lanes per (candidate, segment), one per leg (base replicated, what the
+ * eliminated legs add to it summed across the four lanes): lower latency for batches that
  * leave most SIMDs idle, more instructions in total.  Same layout; equal to spi_rollout_cost up
  * to float rounding (the order of the legs' sums differs). */
 int spi_rollout_cost_legs(const SpiSimArgs* sim, const SpiCostArgs* cost, const float* params_dev, int ld,
@@ -260,8 +262,8 @@ int spi_cem_sample(const float* mean_dev, const float* std_dev, const float* lo_
                    int n, unsigned long long seed, unsigned int iteration, float* theta_dev, int ld,
                    hipStream_t stream);
 
-/* Elite selection + update: sorts (cost, index) of n <= SPI_MAX_CEM_SAMPLES samples in LDS
- * (bitonic), takes the n_elite lowest, writes new mean/std (std floored at min_std_dev[p],
+/* Elite selection + update: orders n <= SPI_MAX_CEM_SAMPLES samples by (cost, index; NaN as
+ * +inf) in LDS, takes the n_elite lowest, writes new mean/std (std floored at min_std_dev[p],
  * blended with the old moments by alpha: new = alpha*old + (1-alpha)*elite), the best sample
  * and its cost (best_dev [n_param], best_cost_dev [1]: kept if not improved), and
  * elite_idx_dev [n_elite] (may be NULL). */
@@ -445,8 +447,8 @@ int spi_policy_step(const SpiSimArgs* sim, const float* params_dev, int ld, int 
                     const float* states_in_dev, float* states_out_dev, const float* actions_dev, const int* done_dev,
                     int sync_first, float* applied_dev, int* bad_dev, hipStream_t stream);
 
-/* The same step with four lanes per env, one per leg (the base replicated, the legs' articulated
- * inertias summed across the four lanes): about a third of the instructions per lane on the
+/* The same step with four lanes per env, one per leg (the base replicated, what the eliminated
+ * legs add to it summed across the four lanes): about a third of the instructions per lane on the
  * critical path, for batches too small to fill the GPU with one env per lane.  Same arguments
  * and results up to float rounding (the order of the legs' sums differs). */
 int spi_policy_step_legs(const SpiSimArgs* sim, const float* params_dev, int ld, int n_env, int group,

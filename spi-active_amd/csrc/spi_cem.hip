@@ -1,5 +1,6 @@
 // Cross-entropy method on device: Gaussian sampling (Philox4x32-10 + Box-Muller), elite
-// selection by an LDS bitonic sort, and the elite-moment update.  Replaces the Optuna
+// selection (counting passes over the costs, or an LDS sort where the elites are many), and the
+// elite-moment update.  Replaces the Optuna
 // samplers of the reference (algo/active_sysid.yaml:20 CmaEsSampler, mass_opt.py:216
 // TPESampler) behind the same ask -> evaluate -> tell loop (active_sysid.py:196-217).
 #include <hip/hip_runtime.h>

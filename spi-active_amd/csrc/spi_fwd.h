@@ -2,7 +2,7 @@
 // eliminated in closed form in its hip frame.  Same model, contact law and integrator as
 // spi_dyn.h in two thirds of its instructions: a rollout lane is bound by VALU issue, so the
 // algebra is what its time consists of (3,546 FLOP per sub-interval against 5,293; vector
-// instructions 3,399 -> 2,180).
+// instructions 3,424 -> 2,222 by the counters).
 //
 // What the leg's structure gives (hip axis x; thigh and calf axes both y; the thigh's origin
 // lies on its own axis through the hip origin O, so every y offset can be absorbed into the
@@ -21,7 +21,7 @@
 //     k = -s (2 wy + s), at p from that point.  No per-link velocity or force is formed, and
 //     with the base's proper acceleration dv/dt + w x v - g as the unknown, none depends on v.
 // Measured on 4096 candidates x 256 segments x H 20 (rollout_cost_kernel): 31.6 -> 23.2 ms by the
-// algebra, -> 16.3 ms with two waves per SIMD (end_leg below, LaneLds in spi_kernels.hip).  Error
+// algebra, -> 16.8 ms with two waves per SIMD (end_leg below, LaneLds in spi_kernels.hip).  Error
 // of the costs against 64 bits: 2.2e-6 before, 2.0e-6 after.
 #pragma once
 #include "spi_dyn.h"
@@ -202,8 +202,8 @@ SPI_HD Real spi_fma(Real a, Real b, Real c) {
 // penetration is summed from the largest terms down: they cancel to the millimetre, and the
 // stiffness turns each 1e-8 m of rounding into 5e-4 N.
 // SKIP: lanes off the ground skip the block.  One rollout per lane, a wave holds candidates of one
-// segment, whose foot is off the ground together (4096 x 256 x H 20: 16.3 ms, 17.1 without the
-// branch); four lanes per rollout, a wave nearly always has a foot down and the skip only costs
+// segment, whose foot is off the ground together (4096 x 256 x H 20 on one box: 16.3 ms, 17.1 without
+// the branch); four lanes per rollout, a wave nearly always has a foot down and the skip only costs
 // its zeroed results (256 x 64 x H 5: 131 us, 126 without).
 struct FootLoad { V3 f; Real mx, mz, y2, y3; };
 template <bool SKIP, class C>

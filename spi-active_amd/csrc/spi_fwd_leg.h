@@ -2,8 +2,8 @@
 // same instruction stream with the leg's constants in registers; the four legs' contributions
 // to the base are summed by DPP quad steps and the base is solved identically in the four lanes.
 // For batches that leave most SIMDs idle, where one wavefront's instruction count is the time:
-// 1,010 -> 790 vector instructions per sub-interval against the articulated-body form; 256 candidates
-// x 64 segments x H 5 (one wave on every SIMD) 163 -> 134 us.
+// 1,010 -> 770 vector instructions per sub-interval against the articulated-body form; 256 candidates
+// x 64 segments x H 5 (one wave on every SIMD) 163 -> 126 us.
 #pragma once
 #include "spi_dyn_leg.h"
 #include "spi_fwd.h"

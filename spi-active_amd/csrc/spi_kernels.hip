@@ -131,9 +131,9 @@ __device__ __forceinline__ unsigned int rollout_lane(const SpiSimArgs& a, const 
 }
 
 // One workgroup = one segment x 256 candidates; parameters are read coalesced from the SoA array,
-// the segment record through the scalar cache.  Bound by VALU issue: 244 registers (two waves per
+// the segment record through the scalar cache.  Bound by VALU issue: 245 registers (two waves per
 // SIMD), no spills, no copies between register files.  4096 candidates x 256 segments x H 20:
-// 31.6 ms with the articulated-body step at 438 registers, 16.3 ms now (73.0 TFLOP/s of the
+// 31.6 ms with the articulated-body step at 438 registers, 16.8 ms now (70.8 TFLOP/s of the
 // algorithm's own 56,739 FLOP per control step).
 __global__ __launch_bounds__(kRolloutThreads, 2) void rollout_cost_kernel(
     SpiSimArgs a, SpiCostArgs cost, const float* __restrict__ par, int ld, int n_cand,

@@ -7,7 +7,7 @@
 // tile, rows of X and the weight rows staged through LDS in K chunks of 64 (even columns, then odd
 // ones, 65 words per row, so the operand reads of a wavefront hit 64 distinct banks).  Strict IEEE
 // float32 (no fast-math).
-// The actor (900 -> 512 -> 256 -> 128 -> 12): 2048 rows 63 -> 54 us, 16384 rows 222 -> 205 us.
+// The actor (900 -> 512 -> 256 -> 128 -> 12): 2048 rows 63 -> 54 us, 16384 rows 222 -> 200 us.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -352,7 +352,7 @@ __device__ __forceinline__ void tile_of(int id, int n_tiles, int n_col, int* row
 // order does not depend on the source: dense and ring input give the same bits.
 // A result that is not finite (an infinite or NaN operand, or one of 2^112 and more, has no finite
 // parts) is formed again on the float32 pipe, by its wavefront together: 16 bad rows of 2048 1220 us
-// with a loop per element, 88 us so
+// with a loop per element, 90 us so
 // (66 where every batch took the float32 pipe).
 constexpr int kSpTile = 64, kSpK = 32;
 constexpr int kSpGroupTiles = 256, kSpWideTiles = 1024;   // tiles of 64 x 64
@@ -589,9 +589,10 @@ int launch_linear(const float* X, int ldx, const RingSrc& rs, int M, int K, cons
   const bool ring4 = rs.ring && rs.ld % 4 == 0 && aligned16(rs.ring);
   if (N >= kSpTile && K >= 2 * kSpK && wvec && xvec) {
     const long long rows = (M + kSpTile - 1) / kSpTile, tiles = rows * ((N + kSpTile - 1) / kSpTile);
-    // A tile per CU or less: two groups share its chunks (900 -> 512 at 2048 rows, 256 tiles: 23.5
-    // us, 26.3 with one; at 4096 rows 46.7, 37.0 with one).  From two 64 x 128 tiles per CU on:
-    // those (16384 rows 122 us, 136 with 64 x 64; 4096 rows, one per CU, 39.7 against 37.0).
+    // us of a layer 900 -> 512, two groups / one group per 64 x 64 tile / 64 x 128 tiles / the float32
+    // pipe.  A tile per CU or less, two groups share its chunks: 16 rows 20.5 / 23.7 / 37 / 25.5, 256 rows 21.4 / 24.6 / 39 / 26.8, 2048 rows (256 tiles) 24.5 / 26.3 / 40 / 28.4.  Above, one: 4096
+    // rows 44.7 / 40.0 / 43.0 / 44.1.  From two 64 x 128 tiles per CU on, those: 8192 rows 85 / 72 / 68 / 78,
+    // 16384 rows 168 / 134 / 127 / 131.
     const int shape = tiles <= kSpGroupTiles ? 0 : tiles < kSpWideTiles ? 1 : 2;
 #define SPI_SP_G(E, S, NN, G) \
   linear_split_kernel<E, S, NN, G><<<static_cast<int>(rows * ((N + kSpTile * NN - 1) / (kSpTile * NN))), 256 * G, 0, stream>>>( \

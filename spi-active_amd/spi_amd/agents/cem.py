@@ -7,7 +7,7 @@ kernel launches and never synchronises with the host:
 
   spi_cem_sample   theta = clamp(mean + std * z, lo, hi), z from Philox4x32-10 + Box-Muller
   (evaluate)       any batched objective, e.g. spi_rollout_cost + spi_reduce_segments
-  spi_cem_update   bitonic sort of (cost, index) in LDS, elite moments, best-so-far
+  spi_cem_update   selection of the elites by (cost, index) in LDS, their moments, best-so-far
 
 Parameters with ``std0 == 0`` and ``min_std == 0`` stay fixed at their mean.
 """
