@@ -10,6 +10,23 @@
 
 namespace SPI_DYN_NS {
 
+// Parameters of lane i from their rows [25][ld], the base with the legs' axial mass.
+__device__ __forceinline__ LaneParams load_params(const float* __restrict__ par, int ld, int i) {
+  LaneParams lp;
+  lp.base = base_with_legs(make_base_inertia(par[0 * ld + i], par[1 * ld + i], par[2 * ld + i], par[3 * ld + i],
+                                             par[4 * ld + i], par[5 * ld + i], par[6 * ld + i], par[7 * ld + i],
+                                             par[8 * ld + i], par[9 * ld + i]));
+#pragma unroll
+  for (int l = 0; l < 4; ++l) {
+    lp.kp_s[l] = par[(10 + l) * ld + i];
+    lp.kd_s[l] = par[(14 + l) * ld + i];
+    lp.fric[l] = par[(18 + l) * ld + i];
+  }
+#pragma unroll
+  for (int g = 0; g < 3; ++g) lp.motor[g] = par[(22 + g) * ld + i];
+  return lp;
+}
+
 struct ElimTable { LegC<float> k[4]; };
 constexpr ElimTable elim_table() { return ElimTable{{leg_c<float>(0), leg_c<float>(1), leg_c<float>(2), leg_c<float>(3)}}; }
 static __constant__ ElimTable kElimTab = elim_table();

@@ -33,23 +33,6 @@ int launch_check(const char* what) { return hip_check(hipGetLastError(), what); 
 using spi_launch::apply_segment_gains;
 using spi_launch::xcd_remap;
 
-// Parameters of lane i, the base with the legs' axial mass (spi_fwd.h).
-__device__ __forceinline__ LaneParams load_params(const float* __restrict__ par, int ld, int i) {
-  LaneParams lp;
-  lp.base = make_base_inertia(par[0 * ld + i], par[1 * ld + i], par[2 * ld + i], par[3 * ld + i], par[4 * ld + i],
-                              par[5 * ld + i], par[6 * ld + i], par[7 * ld + i], par[8 * ld + i], par[9 * ld + i]);
-  lp.base = base_with_legs(lp.base);
-#pragma unroll
-  for (int l = 0; l < 4; ++l) {
-    lp.kp_s[l] = par[(10 + l) * ld + i];
-    lp.kd_s[l] = par[(14 + l) * ld + i];
-    lp.fric[l] = par[(18 + l) * ld + i];
-  }
-#pragma unroll
-  for (int g = 0; g < 3; ++g) lp.motor[g] = par[(22 + g) * ld + i];
-  return lp;
-}
-
 using spi_launch::finite_bits;
 using spi_launch::lane_params_valid;
 
@@ -484,10 +467,6 @@ __global__ __launch_bounds__(256) void fim_rollout_kernel(SpiSimArgs a, const fl
   if (active && member == 0) fim[group] = acc;
 }
 
-bool sim_args_ok(const SpiSimArgs* a) {
-  return a && a->dt > 0.f && a->decimation >= 1 && a->decimation <= 64 && a->substeps >= 1 && a->substeps <= 64 &&
-         a->motor_model >= 0 && a->motor_model <= 3 && a->state_limit > 0.f;
-}
 
 }  // namespace
 
@@ -519,7 +498,7 @@ int spi_rigid_body_states(const float* root_dev, const float* dof_state_dev, int
 
 int spi_compute_torques(const SpiSimArgs* sim, const float* params_dev, int ld, int n, const float* actions_dev,
                         const float* dof_state_dev, float* torques_dev, hipStream_t stream) {
-  if (!sim_args_ok(sim)) return fail(SPI_ERR_INVALID_ARG, "spi_compute_torques: invalid SpiSimArgs");
+  if (!spi_launch::sim_args_ok(sim)) return fail(SPI_ERR_INVALID_ARG, "spi_compute_torques: invalid SpiSimArgs");
   if (n < 0 || ld < n || !params_dev || !actions_dev || !dof_state_dev || !torques_dev)
     return fail(SPI_ERR_INVALID_ARG, "spi_compute_torques: bad sizes or null pointer");
   if (n == 0) return SPI_OK;
@@ -540,7 +519,7 @@ int spi_fd_fim_trace(const float* root_dev, const float* dof_state_dev, const fl
 
 int spi_rollout_cost(const SpiSimArgs* sim, const SpiCostArgs* cost, const float* params_dev, int ld, int n_cand,
                      const float* seg_dev, int n_seg, int horizon, float* cost_seg_dev, hipStream_t stream) {
-  if (!sim_args_ok(sim) || !cost || (cost->mode != SPI_COST_TRACKING && cost->mode != SPI_COST_REFERENCE))
+  if (!spi_launch::sim_args_ok(sim) || !cost || (cost->mode != SPI_COST_TRACKING && cost->mode != SPI_COST_REFERENCE))
     return fail(SPI_ERR_INVALID_ARG, "spi_rollout_cost: invalid SpiSimArgs/SpiCostArgs");
   if (n_cand < 0 || n_seg < 0 || horizon < 1 || ld < n_cand || !params_dev || !seg_dev || !cost_seg_dev)
     return fail(SPI_ERR_INVALID_ARG, "spi_rollout_cost: bad sizes or null pointer");
@@ -562,7 +541,7 @@ int spi_rollout_cost(const SpiSimArgs* sim, const SpiCostArgs* cost, const float
 int spi_rollout_cost_legs(const SpiSimArgs* sim, const SpiCostArgs* cost, const float* params_dev, int ld,
                           int n_cand, const float* seg_dev, int n_seg, int horizon, float* cost_seg_dev,
                           hipStream_t stream) {
-  if (!sim_args_ok(sim) || !cost || (cost->mode != SPI_COST_TRACKING && cost->mode != SPI_COST_REFERENCE))
+  if (!spi_launch::sim_args_ok(sim) || !cost || (cost->mode != SPI_COST_TRACKING && cost->mode != SPI_COST_REFERENCE))
     return fail(SPI_ERR_INVALID_ARG, "spi_rollout_cost_legs: invalid SpiSimArgs/SpiCostArgs");
   if (n_cand < 0 || n_seg < 0 || horizon < 1 || ld < n_cand || !params_dev || !seg_dev || !cost_seg_dev)
     return fail(SPI_ERR_INVALID_ARG, "spi_rollout_cost_legs: bad sizes or null pointer");
@@ -583,7 +562,7 @@ int spi_rollout_cost_legs(const SpiSimArgs* sim, const SpiCostArgs* cost, const 
 int spi_fim_rollout(const SpiSimArgs* sim, const float* params_dev, int ld, int n_group, int n_param,
                     const float* init_dev, const float* actions_dev, int n_steps, float delta, int ksync,
                     int ksync_mode, float* fim_dev, hipStream_t stream) {
-  if (!sim_args_ok(sim)) return fail(SPI_ERR_INVALID_ARG, "spi_fim_rollout: invalid SpiSimArgs");
+  if (!spi_launch::sim_args_ok(sim)) return fail(SPI_ERR_INVALID_ARG, "spi_fim_rollout: invalid SpiSimArgs");
   if (n_group < 0 || n_param < 1 || n_param + 1 > 64 || n_steps < 1 || !(delta != 0.0f) ||
       (ksync_mode != 0 && ksync_mode != 1) || !params_dev || !init_dev || !actions_dev || !fim_dev)
     return fail(SPI_ERR_INVALID_ARG, "spi_fim_rollout: bad arguments");
@@ -604,7 +583,7 @@ int spi_fim_rollout(const SpiSimArgs* sim, const float* params_dev, int ld, int 
 int spi_batch_rollout_cost(const SpiSimArgs* sim, const SpiBatchProblem* probs_dev, const long long* task_prefix_dev,
                            int n_prob, long long n_tasks, int max_horizon, int block, int unroll, int n_blocks,
                            unsigned long long* queue_dev, hipStream_t stream) {
-  if (!sim_args_ok(sim)) return fail(SPI_ERR_INVALID_ARG, "spi_batch_rollout_cost: invalid SpiSimArgs");
+  if (!spi_launch::sim_args_ok(sim)) return fail(SPI_ERR_INVALID_ARG, "spi_batch_rollout_cost: invalid SpiSimArgs");
   if (n_prob < 1 || n_tasks < 0 || max_horizon < 1 || n_blocks < 1 || !probs_dev || !task_prefix_dev || !queue_dev)
     return fail(SPI_ERR_INVALID_ARG, "spi_batch_rollout_cost: bad arguments");
   if (n_tasks == 0) return SPI_OK;

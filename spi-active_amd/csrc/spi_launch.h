@@ -6,6 +6,12 @@
 
 namespace spi_launch {
 
+// Simulation settings that the kernels can run.
+inline bool sim_args_ok(const SpiSimArgs* a) {
+  return a && a->dt > 0.f && a->decimation >= 1 && a->decimation <= 64 && a->substeps >= 1 && a->substeps <= 64 &&
+         a->motor_model >= 0 && a->motor_model <= 3 && a->state_limit > 0.f;
+}
+
 // Recorded PD gains of segment s: when the cost settings carry a per-segment gain table, the
 // kernel's copy of the simulation settings runs the PD law with that segment's (kp, kd) on
 // all 12 joints (scripts/eval.py:192-201 sets env.p_gains/d_gains from the recorded

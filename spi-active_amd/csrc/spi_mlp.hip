@@ -590,9 +590,10 @@ int launch_linear(const float* X, int ldx, const RingSrc& rs, int M, int K, cons
   if (N >= kSpTile && K >= 2 * kSpK && wvec && xvec) {
     const long long rows = (M + kSpTile - 1) / kSpTile, tiles = rows * ((N + kSpTile - 1) / kSpTile);
     // us of a layer 900 -> 512, two groups / one group per 64 x 64 tile / 64 x 128 tiles / the float32
-    // pipe.  A tile per CU or less, two groups share its chunks: 16 rows 20.5 / 23.7 / 37 / 25.5, 256 rows 21.4 / 24.6 / 39 / 26.8, 2048 rows (256 tiles) 24.5 / 26.3 / 40 / 28.4.  Above, one: 4096
-    // rows 44.7 / 40.0 / 43.0 / 44.1.  From two 64 x 128 tiles per CU on, those: 8192 rows 85 / 72 / 68 / 78,
-    // 16384 rows 168 / 134 / 127 / 131.
+    // pipe.  A tile per CU or less, two groups share its chunks: 16 rows 20.5 / 23.7 / 37 / 25.5, 256 rows
+    // 21.4 / 24.6 / 39 / 26.8, 2048 rows (256 tiles) 24.5 / 26.3 / 40 / 28.4.  Above, one: 4096 rows 44.7 /
+    // 40.0 / 43.0 / 44.1.  From two 64 x 128 tiles per CU on, those: 8192 rows 85 / 72 / 68 / 78, 16384
+    // rows 168 / 134 / 127 / 131.
     const int shape = tiles <= kSpGroupTiles ? 0 : tiles < kSpWideTiles ? 1 : 2;
 #define SPI_SP_G(E, S, NN, G) \
   linear_split_kernel<E, S, NN, G><<<static_cast<int>(rows * ((N + kSpTile * NN - 1) / (kSpTile * NN))), 256 * G, 0, stream>>>( \

@@ -38,23 +38,6 @@ __constant__ int kDim[kKeys] = {12, 3, 4, 1, 2, 1, 1, 1, 4, 2, 2, 12, 12, 3};
 constexpr int kOffHost[kKeys] = {0, 12, 15, 19, 20, 22, 23, 24, 25, 29, 31, 33, 45, 57};
 constexpr int kDimHost[kKeys] = {12, 3, 4, 1, 2, 1, 1, 1, 4, 2, 2, 12, 12, 3};
 
-// Parameters of env i, the base with the legs' axial mass (spi_fwd.h).
-__device__ __forceinline__ LaneParams load_lane(const float* __restrict__ par, int ld, int i) {
-  LaneParams lp;
-  lp.base = make_base_inertia(par[0 * ld + i], par[1 * ld + i], par[2 * ld + i], par[3 * ld + i], par[4 * ld + i],
-                              par[5 * ld + i], par[6 * ld + i], par[7 * ld + i], par[8 * ld + i], par[9 * ld + i]);
-  lp.base = base_with_legs(lp.base);
-#pragma unroll
-  for (int l = 0; l < 4; ++l) {
-    lp.kp_s[l] = par[(10 + l) * ld + i];
-    lp.kd_s[l] = par[(14 + l) * ld + i];
-    lp.fric[l] = par[(18 + l) * ld + i];
-  }
-#pragma unroll
-  for (int g = 0; g < 3; ++g) lp.motor[g] = par[(22 + g) * ld + i];
-  return lp;
-}
-
 // v expressed in the frame of the unit quaternion (x, y, z, w) (torch_utils.py quat_rotate_inverse).
 __device__ __forceinline__ void quat_rotate_inverse(float qx, float qy, float qz, float qw, float vx, float vy,
                                                     float vz, float* o) {
@@ -80,7 +63,7 @@ __global__ __launch_bounds__(kPolThreads) void policy_step_kernel(SpiSimArgs a, 
                                                                   float* __restrict__ applied, int* __restrict__ bad) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const LaneParams lp = load_lane(par, ld, i);
+  const LaneParams lp = load_params(par, ld, i);
   const float* src = s_in + static_cast<size_t>(i) * SPI_STATE_DIM;
   State st;
   state_from_root(st, src, src + 13, src + 25, 1);

@@ -6,6 +6,7 @@
 #include <cstdio>
 
 #include "spi_fwd_leg.h"
+#include "spi_launch.h"
 
 using namespace spi;
 
@@ -14,23 +15,6 @@ namespace {
 int rfail(int code, const char* msg) {
   spi_set_error(msg);
   return code;
-}
-
-// Parameters of lane i, the base with the legs' axial mass (spi_fwd.h).
-__device__ __forceinline__ LaneParams load_params(const float* __restrict__ par, int ld, int i) {
-  LaneParams lp;
-  lp.base = base_with_legs(make_base_inertia(par[0 * ld + i], par[1 * ld + i], par[2 * ld + i], par[3 * ld + i],
-                                             par[4 * ld + i], par[5 * ld + i], par[6 * ld + i], par[7 * ld + i],
-                                             par[8 * ld + i], par[9 * ld + i]));
-#pragma unroll
-  for (int l = 0; l < 4; ++l) {
-    lp.kp_s[l] = par[(10 + l) * ld + i];
-    lp.kd_s[l] = par[(14 + l) * ld + i];
-    lp.fric[l] = par[(18 + l) * ld + i];
-  }
-#pragma unroll
-  for (int g = 0; g < 3; ++g) lp.motor[g] = par[(22 + g) * ld + i];
-  return lp;
 }
 
 __global__ __launch_bounds__(256) void physics_step_kernel(SpiSimArgs a, const float* __restrict__ par, int ld,
@@ -150,10 +134,6 @@ __global__ __launch_bounds__(256) void simulate_kernel(SpiSimArgs a, const float
   }
 }
 
-bool sim_args_ok(const SpiSimArgs* a) {
-  return a && a->dt > 0.f && a->decimation >= 1 && a->decimation <= 64 && a->substeps >= 1 && a->substeps <= 64 &&
-         a->motor_model >= 0 && a->motor_model <= 3 && a->state_limit > 0.f;
-}
 int launched() {
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? SPI_OK : rfail(SPI_ERR_HIP, hipGetErrorString(e));
@@ -165,7 +145,7 @@ extern "C" {
 
 int spi_physics_step(const SpiSimArgs* sim, const float* params_dev, int ld, int n, float* root_dev,
                      float* dof_state_dev, const float* torques_dev, float* foot_force_dev, hipStream_t stream) {
-  if (!sim_args_ok(sim)) return rfail(SPI_ERR_INVALID_ARG, "spi_physics_step: invalid SpiSimArgs");
+  if (!spi_launch::sim_args_ok(sim)) return rfail(SPI_ERR_INVALID_ARG, "spi_physics_step: invalid SpiSimArgs");
   if (n < 0 || ld < n || !params_dev || !root_dev || !dof_state_dev || !torques_dev)
     return rfail(SPI_ERR_INVALID_ARG, "spi_physics_step: bad sizes or null pointer");
   if (n == 0) return SPI_OK;
@@ -181,7 +161,7 @@ int spi_physics_step(const SpiSimArgs* sim, const float* params_dev, int ld, int
 int spi_forward_dynamics(const SpiSimArgs* sim, const float* params_dev, int ld, int n, const float* root_dev,
                          const float* dof_state_dev, const float* torques_dev, float* acc_dev, float* foot_force_dev,
                          hipStream_t stream) {
-  if (!sim_args_ok(sim)) return rfail(SPI_ERR_INVALID_ARG, "spi_forward_dynamics: invalid SpiSimArgs");
+  if (!spi_launch::sim_args_ok(sim)) return rfail(SPI_ERR_INVALID_ARG, "spi_forward_dynamics: invalid SpiSimArgs");
   if (n < 0 || ld < n || !params_dev || !root_dev || !dof_state_dev || !torques_dev || !acc_dev)
     return rfail(SPI_ERR_INVALID_ARG, "spi_forward_dynamics: bad sizes or null pointer");
   if (n == 0) return SPI_OK;
@@ -192,7 +172,7 @@ int spi_forward_dynamics(const SpiSimArgs* sim, const float* params_dev, int ld,
 
 int spi_simulate(const SpiSimArgs* sim, const float* params_dev, int ld, int n, const float* init_dev,
                  const float* actions_dev, int n_steps, float* states_dev, hipStream_t stream) {
-  if (!sim_args_ok(sim)) return rfail(SPI_ERR_INVALID_ARG, "spi_simulate: invalid SpiSimArgs");
+  if (!spi_launch::sim_args_ok(sim)) return rfail(SPI_ERR_INVALID_ARG, "spi_simulate: invalid SpiSimArgs");
   if (n < 0 || ld < n || n_steps < 0 || !params_dev || !init_dev || !actions_dev || !states_dev)
     return rfail(SPI_ERR_INVALID_ARG, "spi_simulate: bad sizes or null pointer");
   if (n == 0 || n_steps == 0) return SPI_OK;
